@@ -133,6 +133,12 @@ struct MomArgs {
     const double* obs;
     double* part;      // blocks x P x kOPartRow (k_o_partial)
     const double* w;   // per-sample weights (exact enumeration); nullptr: 1
+    // basic RBM without O in memory (T non-null): states, tanh rows and the
+    // Pfaffian block S x (P - P_rbm)
+    int N, M, P_rbm;
+    const uint64_t* states;
+    const cplx<R>* T;
+    const cplx<R>* Opf;
 };
 constexpr int kOPartRow = 9;
 
@@ -160,6 +166,12 @@ struct SxArgs {
     double* y;           // complex P
     double* pdot;        // per column block: p^H y partial (2 doubles), optional
     const CgStatus* status;
+    // basic RBM without O in memory (T non-null): states, tanh rows and the
+    // Pfaffian block S x (P - P_rbm)
+    int N, M, P_rbm;
+    const uint64_t* states;
+    const cplx<R>* T;
+    const cplx<R>* Opf;
 };
 
 // learned proposal (no counterpart in the reference); see kern_learn.hpp
@@ -404,6 +416,9 @@ hipError_t launch_sx(const SxArgs<R>& a, int blocks, hipStream_t st, hipEvent_t 
                      hipEvent_t e1 = nullptr);
 // ZM (P <= 64*ZM) supported by launch_sx
 int sx_max_params();
+// whether launch_sx and launch_o_partial can form O's entries from the tanh
+// rows of a basic RBM (real size 4 or 8 bytes)
+bool sx_ofree_ok(int real_size, int N, int M, int64_t ld, int npf);
 // waves per k_sx_partial block for an O row length ld (short rows: one
 // block of 16 waves per CU)
 inline int sx_waves(int64_t ld) { return ld <= 128 * 4 ? 16 : 4; }

@@ -18,6 +18,8 @@
 // complex multiply-adds per hidden unit and no transcendental; tanh(theta)
 // is recomputed only for accepted moves.
 #pragma once
+#include <type_traits>
+
 #include "dev_common.hpp"
 #include "kern_api.hpp"
 
@@ -960,10 +962,45 @@ __global__ void __launch_bounds__(256) k_build_O(OArgs<R> a) {
     }
 }
 
+// one aligned 8- or 16-byte load
+__device__ inline cplx<float> ldc(const cplx<float>* p) {
+    const float2 v = *reinterpret_cast<const float2*>(p);
+    return {v.x, v.y};
+}
+__device__ inline cplx<double> ldc(const cplx<double>* p) {
+    const double2 v = *reinterpret_cast<const double2*>(p);
+    return {v.x, v.y};
+}
+template <typename R>
+__device__ inline R fma_r(R a, R b, R c) {
+    if constexpr (sizeof(R) == 4) return __builtin_fmaf(a, b, c);
+    else return __builtin_fma(a, b, c);
+}
+// a b and conj(a) b with the roundings of k_sx_partial's products
+template <typename R>
+__device__ inline cplx<R> cmul_r(cplx<R> a, cplx<R> b) {
+    return {fma_r<R>(a.re, b.re, -(a.im * b.im)), fma_r<R>(a.im, b.re, a.re * b.im)};
+}
+template <typename R>
+__device__ inline cplx<R> cmulc_r(cplx<R> a, cplx<R> b) {
+    return {fma_r<R>(a.re, b.re, a.im * b.im), fma_r<R>(a.re, b.im, -(a.im * b.re))};
+}
+// +-1 from the bit of w shifted up to the sign bit
+template <typename R>
+__device__ inline R pm1(uint32_t w, int up) {
+    const uint32_t s = (w << up) & 0x80000000u;
+    if constexpr (sizeof(R) == 4) return __uint_as_float(s | 0x3F800000u);
+    else return __hiloint2double((int)(s | 0x3FF00000u), 0);
+}
 // ------------------------------------------------------------ moments --
 // per-block partial sums over a chunk of samples: sum O, sum |O|^2,
 // sum E conj(O) (accumulated in double)
-template <typename R>
+// OFREE (basic RBM): O is not read from memory but formed from the tanh rows
+// and the state bits -- the same values, so the same sums bit for bit; a wave
+// then reads a few tanh values per sample instead of 64 entries of O.  Toric
+// 4x4, alpha = 2, 262 144 samples in FP64: 1760 + 1826 us for k_build_O +
+// k_o_partial before, 499 us now (bound by the FP64 pipe).
+template <typename R, bool OFREE>
 __global__ void __launch_bounds__(256) k_o_partial(MomArgs<R> a) {
     // block (chunk b = blockIdx.x, parameters 64 blockIdx.y + lane): sums of
     // O - K, |O - K|^2 with the shift K = the chunk's first O (shifted-data
@@ -974,12 +1011,41 @@ __global__ void __launch_bounds__(256) k_o_partial(MomArgs<R> a) {
     // sum w d im, sum w |d|^2, sum w E conj(O) re, im, sum w, sum w^2];
     // k_o_final merges the chunks.
     __shared__ double red[3][7][64];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    // the wave index, and with it every sample index, in scalar registers:
+    // the weights, energies and states are scalar loads
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int p = (int)blockIdx.y * 64 + lane;
     const bool on = p < a.P;
     const int64_t k0 = (int64_t)blockIdx.x * a.chunk, k1 = k0 + a.chunk < a.S ? k0 + a.chunk : a.S;
     const int pp = on ? p : 0;
-    const cplx<R> o0 = a.O[k0 * a.ld + pp];
+    // OFREE: parameter pp is sigma_j (unit -1), t_unit (j = -1), sigma_j
+    // t_unit, or entry pp - P_rbm of the Pfaffian block
+    int unit = -1, j = -1;
+    if constexpr (OFREE) {
+        const int q = pp - a.N - a.M;
+        if (pp < a.N) j = pp;
+        else if (q < 0) unit = pp - a.N;
+        else if (pp < a.P_rbm) {
+            unit = q / a.N;
+            j = q - unit * a.N;
+        }
+    }
+    const bool pf = OFREE && pp >= a.P_rbm;
+    const int at = pf ? pp - a.P_rbm : unit > 0 ? unit : 0;
+    if (pf) unit = 0;  // (not a visible entry)
+    auto entry = [&](int64_t k) -> cplx<R> {
+        if constexpr (!OFREE) {
+            return a.O[k * a.ld + pp];
+        } else {
+            // one load whatever the entry: a tanh value or a Pfaffian entry
+            const uint64_t w = a.states[k];
+            cplx<R> t = ldc((pf ? a.Opf + k * (a.P - a.P_rbm) : a.T + k * a.M) + at);
+            if (unit < 0) t = {1, 0};
+            const R sg = pm1<R>((uint32_t)((j & 32 ? w >> 32 : w) & (j < 0 ? 0u : ~0u)), 31 - (j & 31));
+            return {sg * t.re, sg * t.im};
+        }
+    };
+    const cplx<R> o0 = entry(k0);
     const double kr = o0.re, ki = o0.im;
     double s0 = 0, s1 = 0, s2 = 0, e0 = 0, e1 = 0, sw = 0, sw2 = 0;
     const int64_t eo = 2 * (int64_t)a.n_groups;
@@ -998,14 +1064,13 @@ __global__ void __launch_bounds__(256) k_o_partial(MomArgs<R> a) {
     };
     int64_t k = k0 + wv;
     for (; k + 12 < k1; k += 16) {  // four rows in flight per wave
-        const cplx<R> o_0 = a.O[k * a.ld + pp], o_1 = a.O[(k + 4) * a.ld + pp];
-        const cplx<R> o_2 = a.O[(k + 8) * a.ld + pp], o_3 = a.O[(k + 12) * a.ld + pp];
+        const cplx<R> o_0 = entry(k), o_1 = entry(k + 4), o_2 = entry(k + 8), o_3 = entry(k + 12);
         add(k, o_0);
         add(k + 4, o_1);
         add(k + 8, o_2);
         add(k + 12, o_3);
     }
-    for (; k < k1; k += 4) add(k, a.O[k * a.ld + pp]);
+    for (; k < k1; k += 4) add(k, entry(k));
     if (wv > 0) {
         double* r = &red[wv - 1][0][lane];
         r[0] = s0;
@@ -1141,6 +1206,311 @@ __global__ void __launch_bounds__(64 * WAVES) k_sx_partial(SxArgs<R> a) {
     }
     cplx<R>* out = a.part + (int64_t)blockIdx.x * a.ld;
     for (int p = threadIdx.x; p < a.ld; p += blockDim.x) out[p] = zs[p];
+}
+
+// ------------------------------------------- S.x without O (basic RBM) --
+// The product of k_sx_partial with the entries of O formed from the tanh row
+// and the state bits (O = sigma_j, t_u, sigma_j t_u; the Pfaffian block is
+// read): the same products and sums in the same order, so the same bits, from
+// S (M complex + 8) bytes instead of S P complex.
+//
+// Why the order is kept: the CG stops at |r|^2 < 1e-16 or at its iteration
+// limit, and on ill-conditioned sample sets (enumerations, fewer samples than
+// parameters) a rounding difference of 1e-16 in this product moves the
+// solution by up to 1e-7.  A matrix-core form (v_mfma_f64_16x16x4, 142 us at
+// the size below) sums in another order and was left out for that.
+//
+// Bound by the FP64 (FP32) vector pipe and the LDS reads: a pair of
+// neighbouring entries of one unit takes 12 operations for the dot product
+// (t b rounded per entry, then +-1 times it added by an FMA, which is exact)
+// and 8 for the accumulation (conj(t) y once per pair).  Toric 4x4 alpha = 2
+// (P = 2144), 262 144 samples, FP64: 2610 us over the 9.0 GB of O, 348 us
+// now; Kitaev 4x4 + Pfaffian (P = 2244), 65 536 samples, FP32: 209 ->
+// 134 us.
+//
+// Each wave takes of_rows of its rows together: one read of x from LDS serves
+// them all, and their reductions overlap; the next rows' loads are issued
+// before the current ones are used.  The tanh value of a lane's pair:
+//  * N = 32 with M a multiple of 32 (B32): the 16 lanes of a DPP row share one
+//    unit per pair, 4 i + (lane / 16) + const for pair i, so lane n of the row
+//    holds the values of pairs n and 16 + n and a row broadcast hands them out
+//    (508 us with LDS reads at the size above);
+//  * otherwise, and for the biases, from the row staged in LDS.
+// The sign is +-1 with the sign bit shifted out of the (wave-uniform) state.
+// rows per step: 4, or 2 where the accumulators leave no registers for more
+// (blocks of 16 waves: 128 per lane; FP64 rows of over 1024 entries)
+template <typename R>
+__host__ __device__ constexpr int of_rows(int waves, int ld) {
+    return waves == 16 || (sizeof(R) == 8 && ld > 1024) ? 2 : 4;
+}
+constexpr int kOfMaxN = 62;  // bit 62 of a masked state word is 0
+// MODE: spins in both halves of the state word, in the low half, B32
+constexpr int kOfWide = 0, kOfN32 = 1, kOfB32 = 2;
+__host__ __device__ inline int of_mode(int N, int M) {
+    return N > 32 ? kOfWide : N == 32 && M % 32 == 0 ? kOfB32 : kOfN32;
+}
+__host__ __device__ inline int of_pad(int ld) { return (ld + 127) / 128 * 128; }
+__host__ __device__ inline int of_xs(int ld, int npf) { return of_pad(ld) + (npf + 1) / 2 * 2; }
+// LDS: x and the waves' rows, then two rows of sums
+template <typename R>
+__host__ __device__ inline size_t of_lds(int ld, int M, int npf, int waves) {
+    const size_t loop = (size_t)of_xs(ld, npf) + (size_t)waves * of_rows<R>(waves, ld) * (M + 1);
+    return (loop > 2 * (size_t)ld ? loop : 2 * (size_t)ld) * sizeof(cplx<R>);
+}
+// basic RBMs whose pairs never straddle two units (even N and M), the biases
+// within the first pair, at least two of the 4-wave blocks' LDS per CU
+template <typename R>
+__host__ __device__ inline bool of_ok(int N, int M, int ld, int npf, int waves) {
+    return N <= kOfMaxN && N % 2 == 0 && M % 2 == 0 && N + M <= 128 &&
+           of_lds<R>(ld, M, npf, waves) <= (waves == 16 ? 163840 : 81920);
+}
+
+// lane n of each 16-lane row to the whole row
+template <int n>
+__device__ inline float row_bcast(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + n, 0xF, 0xF, false));
+}
+template <int n>
+__device__ inline double row_bcast(double v) {
+    return __longlong_as_double(__builtin_amdgcn_update_dpp(0LL, __double_as_longlong(v), 0x150 + n, 0xF, 0xF, false));
+}
+template <int n, typename R>
+__device__ inline cplx<R> row_bcast(cplx<R> v) {
+    return {row_bcast<n>(v.re), row_bcast<n>(v.im)};
+}
+// f(integral_constant<0>) .. f(integral_constant<n - 1>)
+template <int I, int n, typename F>
+__device__ __attribute__((always_inline)) inline void unroll_n(F&& f) {
+    if constexpr (I < n) {
+        f(std::integral_constant<int, I>{});
+        unroll_n<I + 1, n>(f);
+    }
+}
+
+template <typename R, int ZM, int WAVES, int MODE, bool PF>
+__global__ void __launch_bounds__(64 * WAVES, WAVES == 16 ? 4 : 2) k_sx_ofree(SxArgs<R> a) {
+    extern __shared__ __align__(16) char smem[];
+    if (a.status && a.status->done) return;
+    constexpr int RW = of_rows<R>(WAVES, 128 * ZM);
+    constexpr bool B32 = MODE == kOfB32;
+    const int N = a.N, M = a.M, NM = N + M, rs = M + 1;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int npf = a.P - a.P_rbm;
+    // x, zero past the formed entries up to whole pairs of the wave; the
+    // Pfaffian block's x follows
+    const int pw = PF ? a.P_rbm : a.ld, lp = of_pad(a.ld);
+    cplx<R>* b = reinterpret_cast<cplx<R>*>(smem);
+    cplx<R>* tr = b + of_xs(a.ld, npf) + (size_t)wv * RW * rs;  // this wave's rows: tanh, 1
+    for (int p = threadIdx.x; p < lp + npf; p += 64 * WAVES) {
+        const int q = p < lp ? p : a.P_rbm + p - lp;
+        b[p] = q < a.P && (p >= lp || p < pw) ? cplx<R>{(R)a.x[2 * q], (R)a.x[2 * q + 1]} : cplx<R>{0, 0};
+    }
+    if (lane < RW) tr[lane * rs + M] = {1, 0};
+    __syncthreads();
+    const int64_t nwaves = (int64_t)gridDim.x * WAVES;
+    const uint64_t wmask = (((uint64_t)1) << N) - 1;
+    // pair i of the lane: entries p = 2 lane + 128 i and p + 1; lanes past
+    // the formed entries add zeros (x = 0, or t = 0 before the Pfaffian
+    // block), and a sum that starts at +0 keeps its bits.  Pair 0 holds the
+    // biases (N + M <= 128): its places in the row, the spin of its signs (62:
+    // +1); the unit and spin of pair 1 advance by 128 entries from pair to pair
+    const int q0 = 2 * lane - NM;
+    const int e0 = q0 >= 0 ? q0 / N : 2 * lane < N ? M : 2 * lane - N;
+    const int e1 = q0 >= 0 ? e0 : 2 * lane < N ? M : 2 * lane - N + 1;
+    const int ej = q0 >= 0 ? q0 - e0 * N : 2 * lane < N ? 2 * lane : 62;
+    const int j1 = (q0 + 128) % N, du = 128 / N, dj = 128 % N;
+    int uj = (q0 + 128) / N | j1 << 16;
+    cplx<R> z[2 * ZM];
+#pragma unroll
+    for (int i = 0; i < 2 * ZM; i++) z[i] = {0, 0};
+
+    // B32: units of the lane's pairs n = lane % 16 and 16 + n
+    const int ux = (lane >> 4) + 4 * (lane & 15) - NM / 32, uy = ux + 64;
+    constexpr bool two = ZM > 16;  // pairs past the 16th
+    cplx<R> nx[RW], ny[RW];        // the next rows' tanh values
+    uint64_t sw[RW];
+    auto load = [&](int64_t k0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < RW; r++) {
+            const int64_t k = min(k0 + r * nwaves, a.S - 1);  // rows past S are staged but not used
+            sw[r] = a.states[k];
+            nx[r] = ldc(a.T + k * M + (B32 ? min(max(ux, 0), M - 1) : min(lane, M - 1)));
+            if (B32 && two) ny[r] = ldc(a.T + k * M + min(uy, M - 1));
+        }
+    };
+    int64_t k = (int64_t)blockIdx.x * WAVES + wv;
+    if (k < a.S) load(k);
+    for (; k < a.S; k += RW * nwaves) {
+        cplx<R> tx[RW], ty[RW];
+        uint32_t wl[RW], wh[RW];
+        wave_sync();
+#pragma unroll
+        for (int r = 0; r < RW; r++) {
+            const uint64_t w = sw[r] & wmask;
+            wl[r] = (uint32_t)w;
+            wh[r] = (uint32_t)(w >> 32);
+            if constexpr (B32) {
+                tx[r] = nx[r];
+                if (ux >= 0 && ux < M) tr[r * rs + ux] = tx[r];
+                if (two) {
+                    ty[r] = ny[r];
+                    if (uy < M) tr[r * rs + uy] = ty[r];
+                }
+            } else {
+                if (lane < M) tr[r * rs + lane] = nx[r];
+                for (int q = lane + 64; q < M; q += 64)
+                    tr[r * rs + q] = ldc(a.T + min(k + r * nwaves, a.S - 1) * M + q);
+            }
+        }
+        if (k + RW * nwaves < a.S) load(k + RW * nwaves);
+        wave_sync();
+        R s0[RW], s1[RW];  // B32: the lane's spins are the same in every pair
+        if constexpr (B32) {
+#pragma unroll
+            for (int r = 0; r < RW; r++) {
+                s0[r] = pm1<R>(wl[r], 31 - j1);
+                s1[r] = pm1<R>(wl[r], 30 - j1);
+            }
+        }
+        // tanh values and signs of the lane's pair i in row r
+        auto pair = [&](auto ic, int r, int u, int j, cplx<R>& t0, cplx<R>& t1, R& a0, R& a1)
+                        __attribute__((always_inline)) {
+            constexpr int i = decltype(ic)::value;
+            if constexpr (i == 0) {
+                t0 = ldc(tr + r * rs + e0);
+                t1 = ldc(tr + r * rs + e1);
+                const uint32_t h = ej < 32 ? wl[r] : wh[r];
+                a0 = pm1<R>(h, 31 - (ej & 31));
+                a1 = pm1<R>(h, 30 - (ej & 31));
+            } else if constexpr (B32) {
+                t0 = t1 = i < 16 ? row_bcast<i & 15>(tx[r]) : row_bcast<i & 15>(ty[r]);
+                a0 = s0[r];
+                a1 = s1[r];
+            } else {
+                t0 = t1 = ldc(tr + r * rs + u);
+                const uint32_t h = MODE == kOfN32 || j < 32 ? wl[r] : wh[r];
+                a0 = pm1<R>(h, 31 - (j & 31));
+                a1 = pm1<R>(h, 30 - (j & 31));
+            }
+            if constexpr (PF)  // the Pfaffian block's lanes
+                if (2 * lane + 128 * i >= a.P_rbm) t0 = t1 = {0, 0};
+        };
+        int u, j;
+        auto next = [&](int i) __attribute__((always_inline)) {
+            if (B32) return;
+            if (i == 0) {
+                u = uj & 0xFFFF;
+                j = uj >> 16;
+                return;
+            }
+            u = min(u + du, M);  // past the end: x = 0 there
+            j += dj;
+            if (j >= N) {
+                j -= N;
+                u = min(u + 1, M);
+            }
+        };
+        // ---- y_r = O_r . x
+        cplx<R> dot[RW];
+#pragma unroll
+        for (int r = 0; r < RW; r++) dot[r] = {0, 0};
+        unroll_n<0, ZM>([&](auto ic) __attribute__((always_inline)) {
+            constexpr int i = decltype(ic)::value;
+            const int p = 2 * lane + 128 * i;
+            if (128 * i < pw) {
+                const cplx<R> b0 = ldc(b + p), b1 = ldc(b + p + 1);
+#pragma unroll
+                for (int r = 0; r < RW; r++) {
+                    cplx<R> t0, t1;
+                    R a0, a1;
+                    pair(ic, r, u, j, t0, t1, a0, a1);
+                    const cplx<R> f0 = cmul_r(t0, b0), f1 = cmul_r(t1, b1);
+                    dot[r].re = fma_r<R>(a1, f1.re, fma_r<R>(a0, f0.re, dot[r].re));
+                    dot[r].im = fma_r<R>(a1, f1.im, fma_r<R>(a0, f0.im, dot[r].im));
+                }
+            }
+            if constexpr (PF) {
+                if (128 * i + 127 >= a.P_rbm && p >= a.P_rbm && p < a.ld) {
+                    const cplx<R> b0 = b[lp + p - a.P_rbm], b1 = b[lp + p - a.P_rbm + 1];
+#pragma unroll
+                    for (int r = 0; r < RW; r++) {
+                        cplx<R> v0, v1;
+                        load_pair<R>(a.Opf + min(k + r * nwaves, a.S - 1) * npf, p - a.P_rbm, v0, v1);
+                        dot[r] = (dot[r] + cmul_r(v0, b0)) + cmul_r(v1, b1);
+                    }
+                }
+            }
+            next(i);
+        });
+#pragma unroll
+        for (int r = 0; r < RW; r++) {
+            dot[r] = group_csum<64>(dot[r]);
+            if (a.wsx) dot[r] = (R)a.wsx[min(k + r * nwaves, a.S - 1)] * dot[r];
+            if (k + r * nwaves >= a.S) dot[r] = {0, 0};
+        }
+        // ---- z += conj(O_r) y_r, rows in order.  The pairs' tanh values and
+        // places are formed again: kept from the first pass they would take
+        // some 4 ZM RW registers
+        if constexpr (B32) {
+#pragma unroll
+            for (int r = 0; r < RW; r++) {
+                asm volatile("" : "+v"(tx[r].re), "+v"(tx[r].im));
+                if (two) asm volatile("" : "+v"(ty[r].re), "+v"(ty[r].im));
+            }
+        } else {
+            asm volatile("" : "+v"(uj)::"memory");
+        }
+        unroll_n<0, ZM>([&](auto ic) __attribute__((always_inline)) {
+            constexpr int i = decltype(ic)::value;
+            const int p = 2 * lane + 128 * i;
+            if (128 * i < pw) {
+#pragma unroll
+                for (int r = 0; r < RW; r++) {
+                    cplx<R> t0, t1;
+                    R a0, a1;
+                    pair(ic, r, u, j, t0, t1, a0, a1);
+                    const cplx<R> w0 = cmulc_r(t0, dot[r]), w1 = i == 0 ? cmulc_r(t1, dot[r]) : w0;
+                    z[2 * i].re = fma_r<R>(a0, w0.re, z[2 * i].re);
+                    z[2 * i].im = fma_r<R>(a0, w0.im, z[2 * i].im);
+                    z[2 * i + 1].re = fma_r<R>(a1, w1.re, z[2 * i + 1].re);
+                    z[2 * i + 1].im = fma_r<R>(a1, w1.im, z[2 * i + 1].im);
+                }
+            }
+            if constexpr (PF) {
+                if (128 * i + 127 >= a.P_rbm && p >= a.P_rbm && p < a.ld) {
+#pragma unroll
+                    for (int r = 0; r < RW; r++) {
+                        cplx<R> v0, v1;
+                        load_pair<R>(a.Opf + min(k + r * nwaves, a.S - 1) * npf, p - a.P_rbm, v0, v1);
+                        z[2 * i] = z[2 * i] + cmulc_r(v0, dot[r]);
+                        z[2 * i + 1] = z[2 * i + 1] + cmulc_r(v1, dot[r]);
+                    }
+                }
+            }
+            next(i);
+        });
+    }
+    const int ld = a.ld;
+    // the waves add up in LDS in order, as in k_sx_partial
+    __syncthreads();
+    cplx<R>* zs = b + ld;
+    for (int p = threadIdx.x; p < ld; p += 64 * WAVES) zs[p] = {0, 0};
+    __syncthreads();
+    for (int w = 0; w < WAVES; w++) {
+        if (wv == w) {
+#pragma unroll
+            for (int i = 0; i < ZM; i++) {
+                int p = 2 * lane + 128 * i;
+                if (p < ld) {
+                    zs[p] = zs[p] + z[2 * i];
+                    zs[p + 1] = zs[p + 1] + z[2 * i + 1];
+                }
+            }
+        }
+        __syncthreads();
+    }
+    cplx<R>* out = a.part + (int64_t)blockIdx.x * ld;
+    for (int p = threadIdx.x; p < ld; p += 64 * WAVES) out[p] = zs[p];
 }
 
 // sums the block partials of one chunk of blocks, in FP64

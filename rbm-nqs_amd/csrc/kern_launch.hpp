@@ -91,12 +91,44 @@ hipError_t launch_build_O(const OArgs<R>& a, hipStream_t st) {
 template <typename R>
 hipError_t launch_o_partial(const MomArgs<R>& a, int blocks, hipStream_t st) {
     if (blocks < 1 || a.P < 1 || a.chunk < 1) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((k_o_partial<R>), dim3(blocks, (unsigned)((a.P + 63) / 64)), dim3(256), 0, st, a);
+    const dim3 grid(blocks, (unsigned)((a.P + 63) / 64));
+    if (a.T) hipLaunchKernelGGL((k_o_partial<R, true>), grid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((k_o_partial<R, false>), grid, dim3(256), 0, st, a);
     return hipGetLastError();
 }
 
+// the same grid, waves and order as sx_one
+template <typename R, int ZM, int WAVES, int MODE, bool PF>
+static hipError_t sx_ofree_go(const SxArgs<R>& a, int blocks, hipStream_t st) {
+    const int npf = a.P - a.P_rbm;
+    const size_t lds = of_lds<R>(a.ld, a.M, npf, WAVES);
+    if (!of_ok<R>(a.N, a.M, a.ld, npf, WAVES)) return hipErrorInvalidValue;
+    if (lds > 65536) {
+        hipError_t e = hipFuncSetAttribute((const void*)k_sx_ofree<R, ZM, WAVES, MODE, PF>,
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL((k_sx_ofree<R, ZM, WAVES, MODE, PF>), dim3(blocks), dim3(64 * WAVES), lds, st, a);
+    return hipGetLastError();
+}
+template <typename R, int ZM, int WAVES>
+static hipError_t sx_ofree(const SxArgs<R>& a, int blocks, hipStream_t st) {
+    const bool pf = a.P > a.P_rbm;
+    const int mode = of_mode(a.N, a.M);
+    // N >= 32 has P >= 1088, in blocks of 4 waves; the Pfaffian factor N <= 32
+    if constexpr (WAVES == 4) {
+        if (mode == kOfB32)
+            return pf ? sx_ofree_go<R, ZM, WAVES, kOfB32, true>(a, blocks, st)
+                      : sx_ofree_go<R, ZM, WAVES, kOfB32, false>(a, blocks, st);
+        if (mode == kOfWide) return pf ? hipErrorInvalidValue : sx_ofree_go<R, ZM, WAVES, kOfWide, false>(a, blocks, st);
+    }
+    if (mode != kOfN32) return hipErrorInvalidValue;
+    return pf ? sx_ofree_go<R, ZM, WAVES, kOfN32, true>(a, blocks, st)
+              : sx_ofree_go<R, ZM, WAVES, kOfN32, false>(a, blocks, st);
+}
 template <typename R, int ZM, int WAVES = 4>
 static hipError_t sx_one(const SxArgs<R>& a, int blocks, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
+    if (a.T) return sx_ofree<R, ZM, WAVES>(a, blocks, st);
     size_t lds = 2 * (size_t)a.ld * sizeof(cplx<R>);
     if (lds > 65536) {
         hipError_t e = hipFuncSetAttribute((const void*)k_sx_partial<R, ZM, WAVES>,

@@ -71,6 +71,13 @@ struct rbmgpu_ctx {
     bool have_chains = false;
     // structured: basic RBM in FP32 without an O matrix (kern_struct.hpp)
     bool structured = false;
+    // ofree: other basic RBMs (FP64, keep_o, Pfaffian factor); moments and S.x
+    // form O's entries from the states and tanh rows (k_sx_ofree,
+    // k_o_partial), the O matrix is built when something reads it
+    // (rbmgpu_get_samples, the explicit S)
+    bool ofree = false;
+    bool o_built = false;  // d_O holds the current sample set (ofree)
+    int64_t o_cap = 0;     // samples d_O has room for (ofree)
     int64_t ld_s = 0;  // structured partial row: [P | sum |t|^2 (M)], even
     // moments
     double *d_part = nullptr, *d_omean = nullptr, *d_ovar = nullptr, *d_eo = nullptr,
@@ -295,7 +302,7 @@ int ensure_samples(rbmgpu_ctx* c, int64_t S) {
     if (int rc = dalloc(ctx, &c->d_states, S * c->nw * sizeof(uint64_t))) return rc;
     if (int rc = dalloc(ctx, &c->d_obs, S * 2 * c->n_groups * sizeof(double))) return rc;
     if (int rc = dalloc(ctx, &c->d_T, S * c->H * 2 * rsize(c))) return rc;
-    if (!c->structured)
+    if (!c->structured && !c->ofree)
         if (int rc = dalloc(ctx, &c->d_O, S * c->ld * 2 * rsize(c))) return rc;
     if (c->pf_rows)
         if (int rc = dalloc(ctx, &c->d_Opf, S * 4 * c->pf_rows * 2 * rsize(c))) return rc;
@@ -588,9 +595,8 @@ int learn_tables(rbmgpu_ctx* c, const int32_t* clusters) {
 }
 
 template <typename R>
-int run_build_O(rbmgpu_ctx* c) {
+int enqueue_build_O(rbmgpu_ctx* c) {
     rbmgpu_ctx* ctx = c;
-    if (c->structured || c->S == 0) return 0;
     OArgs<R> a{};
     a.d = dims(c);
     a.S = c->S;
@@ -604,6 +610,27 @@ int run_build_O(rbmgpu_ctx* c) {
     a.Opf = c->pf_rows ? (const cplx<R>*)c->d_Opf : nullptr;
     a.O = (cplx<R>*)c->d_O;
     HIPCK(launch_build_O<R>(a, c->stream));
+    return 0;
+}
+
+// the O matrix of a new sample set: at once, or not until it is read (ofree)
+template <typename R>
+int run_build_O(rbmgpu_ctx* c) {
+    c->o_built = false;
+    if (c->structured || c->ofree || c->S == 0) return 0;
+    return enqueue_build_O<R>(c);
+}
+
+// ofree: the O matrix of the current sample set, if it is not there yet
+int ensure_O(rbmgpu_ctx* c) {
+    rbmgpu_ctx* ctx = c;
+    if (!c->ofree || c->o_built || c->S == 0) return 0;
+    if (c->S > c->o_cap) {
+        if (int rc = dalloc(ctx, &c->d_O, c->S * c->ld * 2 * rsize(c))) return rc;
+        c->o_cap = c->S;
+    }
+    if (int rc = c->prec == RBMGPU_FP32 ? enqueue_build_O<float>(c) : enqueue_build_O<double>(c)) return rc;
+    c->o_built = true;
     return 0;
 }
 
@@ -1381,6 +1408,14 @@ SxArgs<R> sx_args(rbmgpu_ctx* c, const double* x, double* y, double r1, double r
     a.part = (cplx<R>*)c->d_sxpart;
     a.y = y;
     a.status = st;
+    if (c->ofree) {
+        a.N = c->N;
+        a.M = c->na;
+        a.P_rbm = (int)c->P_rbm;
+        a.states = c->d_states;
+        a.T = (const cplx<R>*)c->d_T;
+        a.Opf = (const cplx<R>*)c->d_Opf;
+    }
     return a;
 }
 
@@ -1438,6 +1473,31 @@ int sx(rbmgpu_ctx* c, const double* x, double* y, double r1, double r2, double r
                                   : run_sx<double>(c, x, y, r1, r2, rd, st, pdot, cg, part);
 }
 
+template <typename R>
+int run_o_partial(rbmgpu_ctx* c, int64_t chunk, int blocks, const double* wts) {
+    rbmgpu_ctx* ctx = c;
+    MomArgs<R> a{};
+    a.S = c->S;
+    a.chunk = chunk;
+    a.P = (int)c->P;
+    a.n_groups = c->n_groups;
+    a.ld = (int)c->ld;
+    a.O = (const cplx<R>*)c->d_O;
+    a.obs = c->d_obs;
+    a.part = c->d_part;
+    a.w = wts;
+    a.P_rbm = (int)c->P_rbm;
+    if (c->ofree) {
+        a.N = c->N;
+        a.M = c->na;
+        a.states = c->d_states;
+        a.T = (const cplx<R>*)c->d_T;
+        a.Opf = (const cplx<R>*)c->d_Opf;
+    }
+    HIPCK(launch_o_partial<R>(a, blocks, c->stream));
+    return 0;
+}
+
 int compute_moments(rbmgpu_ctx* c) {
     rbmgpu_ctx* ctx = c;
     if (c->S == 0) return fail(c, "no samples");
@@ -1492,15 +1552,9 @@ int compute_moments(rbmgpu_ctx* c) {
             if (int rc = dalloc(ctx, &c->d_part, need * sizeof(double))) return rc;
             c->part_cap = need;
         }
-        if (c->prec == RBMGPU_FP32) {
-            MomArgs<float> a{c->S, chunk, (int)c->P, c->n_groups, (int)c->ld, (const cplx<float>*)c->d_O, c->d_obs,
-                             c->d_part, wts};
-            HIPCK(launch_o_partial<float>(a, (int)blocks, c->stream));
-        } else {
-            MomArgs<double> a{c->S, chunk, (int)c->P, c->n_groups, (int)c->ld, (const cplx<double>*)c->d_O, c->d_obs,
-                              c->d_part, wts};
-            HIPCK(launch_o_partial<double>(a, (int)blocks, c->stream));
-        }
+        if (int rc = c->prec == RBMGPU_FP32 ? run_o_partial<float>(c, chunk, (int)blocks, wts)
+                                            : run_o_partial<double>(c, chunk, (int)blocks, wts))
+            return rc;
         if (int rc = zero_async(c, c->d_maxvar, sizeof(double))) return rc;
         hipLaunchKernelGGL(k_o_final, dim3((unsigned)c->P), dim3(256), 0, c->stream, c->d_part, blocks, (int)c->P,
                            c->d_omean, c->d_ovar, c->d_eo, (unsigned long long*)c->d_maxvar);
@@ -1733,6 +1787,7 @@ int build_S_t(rbmgpu_ctx* c, double r1, double r2, double rd, int mode, const do
 
 int build_S(rbmgpu_ctx* c, double r1, double r2, double rd, int mode, const double* reg_dev = nullptr) {
     rbmgpu_ctx* ctx = c;
+    if (int rc = ensure_O(c)) return rc;
     if (c->structured || !c->d_O)
         return fail(c, "explicit S needs the O matrix: set keep_o (gpu.keep_o = true) for the cg-single / direct "
                        "solvers");
@@ -2241,6 +2296,8 @@ int rbmgpu_create(const rbmgpu_config* cfg, rbmgpu_ctx** out) {
                         c->prec == RBMGPU_FP32 && c->nw == 1 && sl > 0 && sl <= c->lds_limit;
         c->ld_s = c->P + c->na + ((c->P + c->na) & 1);
     }
+    c->ofree = !c->structured && c->nsymm == 1 && c->nvb == c->N && c->nw == 1 && c->ld <= sx_max_params() &&
+               sx_ofree_ok((int)rsize(c), c->N, c->na, c->ld, 4 * c->pf_rows);
     c->params.assign(c->P, 0.);
     if (build_weight_tables(c)) return bad(c->err);
     if (cfg->learn_hidden > 0) {  // learned proposal
@@ -2416,6 +2473,7 @@ int rbmgpu_train_epoch(rbmgpu_ctx* c, uint32_t epoch, const rbmgpu_sr_params* sp
             if (g.first == budget) ex = g.second;
         if (ex) {
             HIPCK(hipGraphLaunch(ex, c->stream));
+            c->o_built = c->train_dense == 1;  // the replay's samples; O only if S was built from it
         } else {
             // this epoch runs eagerly (allocating what it needs), then the
             // same body is captured for the following epochs
@@ -2924,6 +2982,8 @@ int rbmgpu_get_samples(const rbmgpu_ctx* cc, uint64_t* states, double* obs, doub
     if (obs) HIPCK(hipMemcpy(obs, c->d_obs, c->S * 2 * c->n_groups * 8, hipMemcpyDeviceToHost));
     if (O) {
         if (c->structured) return fail(c, "the O matrix is not materialised in structured mode (keep_o = 0)");
+        if (int rc = ensure_O(c)) return rc;
+        HIPCK(hipStreamSynchronize(c->stream));
         if (c->prec == RBMGPU_FP64) {
             HIPCK(hipMemcpy2D(O, c->P * 16, c->d_O, c->ld * 16, c->P * 16, c->S, hipMemcpyDeviceToHost));
         } else {
