@@ -112,6 +112,22 @@ struct EvalArgs {
     int n_flips;
 };
 
+// log psi of given states without the Pfaffian factor (kern_logpsi.hip)
+template <typename R>
+struct LogpsiArgs {
+    int64_t n;
+    int N, H, na, ns, nw;
+    int w_lds;  // set by the launcher
+    const uint64_t* states;
+    const cplx<R>* W;
+    const cplx<R>* hb;
+    const cplx<R>* lb;
+    const uint8_t* perm;
+    double* logpsi;
+};
+template <typename R>
+hipError_t launch_logpsi(LogpsiArgs<R> a, int n_cu, hipStream_t st);
+
 template <typename R>
 struct OArgs {
     Dims d;

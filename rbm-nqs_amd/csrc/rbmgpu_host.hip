@@ -1574,6 +1574,9 @@ int ensure_eval(rbmgpu_ctx* c, int64_t n) {
     return 0;
 }
 
+// k_logpsi keeps the symmetry permutations in LDS (at most 64 KiB)
+bool logpsi_tables_fit(const rbmgpu_ctx* c) { return c->nsymm == 1 || (int64_t)c->nsymm * c->N <= 65536; }
+
 template <typename R>
 int run_eval(rbmgpu_ctx* c, const uint64_t* d_states, int64_t n, double* logpsi, double* obs, void* Tout,
              double* ratio, const int32_t* flips, int nf) {
@@ -1602,6 +1605,27 @@ int run_eval(rbmgpu_ctx* c, const uint64_t* d_states, int64_t n, double* logpsi,
                 if (shape_fits(c, kShapes[i]) && (!s.L || kShapes[i].L * kShapes[i].K < s.L * s.K)) s = kShapes[i];
     }
     if (!s.L) return fail(c, "no launch shape for this number of hidden units");
+    // log psi alone, for a caller that reads it: 16 states per tile.  (With
+    // other outputs -- sample sets, exact enumeration, whose weights |psi|^2
+    // the SR solve amplifies -- a group of lanes per state, whose sums keep
+    // their order.)
+    if (logpsi && !obs && !Tout && !ratio && !c->pf_rows && logpsi_tables_fit(c)) {
+        LogpsiArgs<R> la{};
+        la.n = n;
+        la.N = c->N;
+        la.H = c->H;
+        la.na = c->na;
+        la.ns = c->nsymm;
+        la.nw = c->nw;
+        la.states = d_states;
+        la.W = a.t.W;
+        la.hb = a.t.hb;
+        la.lb = a.t.lb;
+        la.perm = a.t.perm;
+        la.logpsi = logpsi;
+        HIPCK(launch_logpsi<R>(la, c->n_cu, c->stream));
+        return 0;
+    }
     int block = pick_block(c, s.L, n);
     a.d = dims(c, block);
     HIPCK(launch_eval<R>(a, s, block, c->stream));
