@@ -417,6 +417,9 @@ __host__ __device__ inline size_t wave_lds_bytes(const Dims& d, int K, int npair
     return (b + 15) & ~(size_t)15;
 }
 hipError_t launch_sample_wave(const SampArgs<float>& a, int K, int block, hipStream_t st);
+// given states (a.states, a.n_samples of them): tanh rows and, with a.obs,
+// local observables through the same tables (k_eval_wave)
+hipError_t launch_eval_wave(const SampArgs<float>& a, int K, int n_cu, hipStream_t st);
 // the Pfaffian factor runs one chain per wavefront
 inline bool shape_ok_pf(Shape s, int N) { return s.L == 64 && N <= kPfMaxN; }
 template <typename R>

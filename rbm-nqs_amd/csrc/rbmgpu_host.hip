@@ -1578,6 +1578,27 @@ int ensure_eval(rbmgpu_ctx* c, int64_t n) {
 bool logpsi_tables_fit(const rbmgpu_ctx* c) { return c->nsymm == 1 || (int64_t)c->nsymm * c->N <= 65536; }
 
 template <typename R>
+int run_logpsi(rbmgpu_ctx* c, const uint64_t* d_states, int64_t n, double* logpsi) {
+    rbmgpu_ctx* ctx = c;
+    const Tabs<R> t = tabs<R>(c);
+    LogpsiArgs<R> a{};
+    a.n = n;
+    a.N = c->N;
+    a.H = c->H;
+    a.na = c->na;
+    a.ns = c->nsymm;
+    a.nw = c->nw;
+    a.states = d_states;
+    a.W = t.W;
+    a.hb = t.hb;
+    a.lb = t.lb;
+    a.perm = t.perm;
+    a.logpsi = logpsi;
+    HIPCK(launch_logpsi<R>(a, c->n_cu, c->stream));
+    return 0;
+}
+
+template <typename R>
 int run_eval(rbmgpu_ctx* c, const uint64_t* d_states, int64_t n, double* logpsi, double* obs, void* Tout,
              double* ratio, const int32_t* flips, int nf) {
     rbmgpu_ctx* ctx = c;
@@ -1609,22 +1630,28 @@ int run_eval(rbmgpu_ctx* c, const uint64_t* d_states, int64_t n, double* logpsi,
     // other outputs -- sample sets, exact enumeration, whose weights |psi|^2
     // the SR solve amplifies -- a group of lanes per state, whose sums keep
     // their order.)
-    if (logpsi && !obs && !Tout && !ratio && !c->pf_rows && logpsi_tables_fit(c)) {
-        LogpsiArgs<R> la{};
-        la.n = n;
-        la.N = c->N;
-        la.H = c->H;
-        la.na = c->na;
-        la.ns = c->nsymm;
-        la.nw = c->nw;
-        la.states = d_states;
-        la.W = a.t.W;
-        la.hb = a.t.hb;
-        la.lb = a.t.lb;
-        la.perm = a.t.perm;
-        la.logpsi = logpsi;
-        HIPCK(launch_logpsi<R>(la, c->n_cu, c->stream));
-        return 0;
+    if (logpsi && !obs && !Tout && !ratio && !c->pf_rows && logpsi_tables_fit(c))
+        return run_logpsi<R>(c, d_states, n, logpsi);
+    if constexpr (sizeof(R) == 4) {
+        // sample sets in FP32: the tanh rows and observables through the wave
+        // sampler's tables (basic RBM: k_eloc's observables), log psi by
+        // k_logpsi.  FP64 sample sets keep the lane-group evaluation: its sums'
+        // order reaches the SR solve, which amplifies a change of rounding.
+        if (Tout == c->d_T && obs == c->d_obs && !ratio && wave_ok(c) && (!logpsi || logpsi_tables_fit(c))) {
+            SampArgs<float> w = samp_args<float>(c, 0, 512, n, 0);
+            const int K = (c->H + 63) / 64;
+            w.npair = c->nsymm > 1 ? c->npair : 0;
+            w.d = wave_dims(c, 512, K, w.npair);
+            w.states = const_cast<uint64_t*>(d_states);
+            if (wave_lds_bytes(w.d, K, w.npair) <= c->lds_limit) {
+                const bool later = eloc_after(c);
+                if (later) w.obs = nullptr;
+                HIPCK(launch_eval_wave(w, K, c->n_cu, c->stream));
+                if (later)
+                    if (int rc = run_eloc(c, n)) return rc;
+                return logpsi ? run_logpsi<float>(c, d_states, n, logpsi) : 0;
+            }
+        }
     }
     int block = pick_block(c, s.L, n);
     a.d = dims(c, block);
