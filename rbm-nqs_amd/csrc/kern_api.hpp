@@ -17,6 +17,7 @@ struct Dims {
     int n_terms, n_rowptr, n_ent;  // sizes of the local-operator tables
     int pf_rows;  // Pfaffian fs_ rows (0: no Pfaffian factor)
     int waves;    // wavefronts per block (per-wave Pfaffian scratch)
+    int pf_full;  // 1: Pfaffian scratch with room for log Pf
 };
 
 // weight tables, all complex R; index k*n_alpha + alpha for the N x n_alpha
@@ -380,8 +381,8 @@ __host__ __device__ inline size_t lds_bytes(const Dims& d) {
     // [sites? | mask? | perm] bytes
     size_t b = ((d.w_lds ? 3 : 2) * (size_t)d.N * d.n_alpha + d.N) * sizeof(cplx<R>);
     if (d.pf_rows)
-        b += (4 * (size_t)d.pf_rows + (size_t)d.waves * pf_scratch<R>(d.N, d.pf_rows)) * sizeof(cplx<R>) +
-             2 * (size_t)d.N * d.N;
+        b += 4 * (size_t)d.pf_rows * sizeof(cplx<R>) + 16 +
+             (size_t)d.waves * pf_scratch<R>(d.N, d.pf_rows, d.pf_full) + 2 * (size_t)d.N * d.N;
     if (d.t_lds) b += (size_t)d.n_ent * 16 + 4 * ((size_t)d.n_rowptr + 3 * d.n_terms) + 8 * (size_t)d.n_terms +
                       d.n_ent;
     b += 8 * (size_t)d.npb;
@@ -420,6 +421,8 @@ hipError_t launch_sample_wave(const SampArgs<float>& a, int K, int block, hipStr
 // given states (a.states, a.n_samples of them): tanh rows and, with a.obs,
 // local observables through the same tables (k_eval_wave)
 hipError_t launch_eval_wave(const SampArgs<float>& a, int K, int n_cu, hipStream_t st);
+// largest block of the FP32 Pfaffian sampler
+constexpr int kPfBlock = 512;
 // the Pfaffian factor runs one chain per wavefront
 inline bool shape_ok_pf(Shape s, int N) { return s.L == 64 && N <= kPfMaxN; }
 template <typename R>

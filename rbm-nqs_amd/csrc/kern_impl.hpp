@@ -69,14 +69,16 @@ __device__ inline Lds<R> stage(const Dims& d, const Tabs<R>& t, const Terms& T, 
     l.pf = {};
     if (d.pf_rows) {
         l.pf.fs = lds_copy(at, t.fs, 4 * (size_t)d.pf_rows);
-        const int sw = pf_scratch<R>(d.N, d.pf_rows);
-        cplx<R>* scr = reinterpret_cast<cplx<R>*>(at) + (size_t)(threadIdx.x >> 6) * sw;
-        at += (size_t)d.waves * sw * sizeof(cplx<R>);
+        const size_t sw = pf_scratch<R>(d.N, d.pf_rows, d.pf_full);
+        at = smem + ((at - smem + 15) & ~(ptrdiff_t)15);
+        cplx<R>* scr = reinterpret_cast<cplx<R>*>(at + (threadIdx.x >> 6) * sw);
+        at += (size_t)d.waves * sw;
         l.pf.N = d.N;
         l.pf.rows = d.pf_rows;
         l.pf.X = scr;
+        l.pf.Xr = reinterpret_cast<double*>(scr);
         l.pf.Xd = reinterpret_cast<cplx<double>*>(scr);
-        l.pf.D = scr + pf_xsize<R>(d.N, d.pf_rows);
+        l.pf.D = scr;
         l.pf.G = l.pf.D + 8 * 32;
         l.pf.F = reinterpret_cast<int*>(l.pf.G + 16 * 16);
     }
@@ -373,8 +375,7 @@ __device__ inline cplx<double> term_ratio(const Dims& d, const Lds<R>& l, const 
     double sc = ::ldexp(1.0, pe);
     cplx<double> out{(double)r.re * sc, (double)r.im * sc};
     if constexpr (PF) {  // times Pf(A(sigma')) / Pf(A(sigma)) (pfaffian.hpp:73-86)
-        PfProp<R, false> pp;
-        cplx<R> q = pf_ratio<R, false>(l.pf, pv, st, fl, mask, ln, pp);
+        cplx<R> q = pf_ratio<R>(l.pf, pv, st, fl, mask, ln);
         out = out * cplx<double>{(double)q.re, (double)q.im};
     }
     return out;
@@ -650,8 +651,11 @@ __device__ inline void eval_obs(const Dims& d, const Lds<R>& l, const Units<R, L
 // bond_flips both ends of a random non-z bond are flipped (taking two
 // slots), else one uniform site; accept if u < |psi'/psi|^2.  At kept
 // steps the local observables and tanh(theta) of the sample are written.
+// With the Pfaffian factor in FP32 up to 8 chains share a block's tables: its
+// LDS lets one block per CU run (Kitaev 4x4), as two wavefronts per SIMD of 256
+// registers; in FP64 one of 512 registers.
 template <typename R, int L, int K, bool PF>
-__global__ void __launch_bounds__(256) k_sample(SampArgs<R> a) {
+__global__ void __launch_bounds__(PF && sizeof(R) == 4 ? kPfBlock : 256) k_sample(SampArgs<R> a) {
     extern __shared__ __align__(16) char smem[];
     const Dims d = a.d;
     Lds<R> l = stage<R>(d, a.t, a.T, a.pb, smem);
@@ -730,8 +734,8 @@ __global__ void __launch_bounds__(256) k_sample(SampArgs<R> a) {
             if (f1 >= 0) bre += (-2 * s1) * l.rb[f1].re;
             lr2 += (R)2.8853900817779268 * bre;  // 2 / ln 2
             if constexpr (PF) {
-                int fl[2] = {f0, f1};
-                cplx<R> q = pf_ratio<R, true>(l.pf, pv, st, fl, f1 >= 0 ? 3 : 1, ln, pp);
+                cplx<R> q = pf_ratio2<R, true>(l.pf, pv, st, __builtin_amdgcn_readfirstlane(f0),
+                                               __builtin_amdgcn_readfirstlane(f1), ln, pp);
                 lr2 += M<R>::log2(norm2(q));
             }
             if (uu < M<R>::exp2(lr2)) {
@@ -1263,28 +1267,6 @@ template <typename R>
 __host__ __device__ inline bool of_ok(int N, int M, int ld, int npf, int waves) {
     return N <= kOfMaxN && N % 2 == 0 && M % 2 == 0 && N + M <= 128 &&
            of_lds<R>(ld, M, npf, waves) <= (waves == 16 ? 163840 : 81920);
-}
-
-// lane n of each 16-lane row to the whole row
-template <int n>
-__device__ inline float row_bcast(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + n, 0xF, 0xF, false));
-}
-template <int n>
-__device__ inline double row_bcast(double v) {
-    return __longlong_as_double(__builtin_amdgcn_update_dpp(0LL, __double_as_longlong(v), 0x150 + n, 0xF, 0xF, false));
-}
-template <int n, typename R>
-__device__ inline cplx<R> row_bcast(cplx<R> v) {
-    return {row_bcast<n>(v.re), row_bcast<n>(v.im)};
-}
-// f(integral_constant<0>) .. f(integral_constant<n - 1>)
-template <int I, int n, typename F>
-__device__ __attribute__((always_inline)) inline void unroll_n(F&& f) {
-    if constexpr (I < n) {
-        f(std::integral_constant<int, I>{});
-        unroll_n<I + 1, n>(f);
-    }
 }
 
 template <typename R, int ZM, int WAVES, int MODE, bool PF>

@@ -5,10 +5,21 @@
 // matrix A(sigma), columns 16h .. 16h + 15 with h = l >> 5: v[q] =
 // inv(i, 16h + q).  Rows i >= N are zero.
 //
-// Per-wave LDS scratch: X (N x N complex double, column-major X[j*N + i])
-// for fresh inverses / Pfaffians, which are always formed in FP64, and as
-// exchange space, D (8 x 32) for the Delta-a rows of a flip set, G (16 x 16)
-// for the small 2m x 2m matrix.
+// Per-wave LDS scratch, one region reused: the real or imaginary parts of a
+// fresh FP64 inverse (N x (N + 1) doubles) while it is transposed, the
+// Pfaffian derivative's sums, and for flip sets of more than two sites D (8 x
+// 32) for the Delta-a rows and G (16 x 16) for the small 2m x 2m matrix.  Where
+// log Pf is asked for (k_eval), the whole matrix (N x N complex double,
+// column-major X[j*N + i]).
+//
+// Cross-lane traffic stays in registers: the 16 lanes of a DPP row read the
+// value of lane q of their row by a row broadcast, rows and halves exchange by
+// v_permlane16_swap / v_permlane32_swap, wave-uniform entries come by
+// v_readlane.  The sampler was bound by the latency of the LDS round trips and
+// fences of these exchanges, at one wavefront per SIMD (20 KB of scratch per
+// wave); Kitaev 4x4 + Pfaffian, 8192 chains x 8 samples, FP32: 119.6 ms before,
+// 49.6 ms now, with the same sums in the same order (the chains are the same
+// state for state).
 //
 // Ratio and update follow pfaffian.cpp:299-397 (Sherman-Morrison-Woodbury):
 // for flips f_0..f_{m-1}, B = [Delta-a columns | unit columns e_{f_k}],
@@ -16,6 +27,8 @@
 // and on acceptance inv += t2 - t2^T with t2 = (inv B) C (inv B)^T / 2,
 // C = antisym(Cinv'^-1).
 #pragma once
+#include <type_traits>
+
 #include "dev_common.hpp"
 
 namespace rbmgpu {
@@ -30,18 +43,16 @@ __device__ inline void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// scratch per wave in complex R entries: X (room for N x N complex double,
-// 256 entries, or 4 rows accumulators), D (8 x 32), G (16 x 16), and 16
-// ints for the flip list (8 complex slots)
+// bytes of a wave's scratch; full: with room for pf_logpf's matrix
 template <typename R>
-__host__ __device__ inline int pf_xsize(int N, int rows) {
-    int x = N * N * (int)(sizeof(cplx<double>) / sizeof(cplx<R>));
-    if (x < 256) x = 256;
-    return 4 * rows > x ? 4 * rows : x;
-}
-template <typename R>
-__host__ __device__ inline int pf_scratch(int N, int rows) {
-    return pf_xsize<R>(N, rows) + 8 * 32 + 16 * 16 + 8;
+__host__ __device__ inline size_t pf_scratch(int N, int rows, int full) {
+    size_t b = (size_t)(8 * 32 + 16 * 16) * sizeof(cplx<R>) + 64;  // D, G, flip list
+    const size_t t = (size_t)N * (N + 1) * sizeof(double), d = 4 * (size_t)rows * sizeof(cplx<R>);
+    const size_t m = full ? (size_t)N * N * sizeof(cplx<double>) : 0;
+    b = b > t ? b : t;
+    b = b > d ? b : d;
+    b = b > m ? b : m;
+    return (b + 15) & ~(size_t)15;
 }
 
 template <typename R>
@@ -49,11 +60,13 @@ struct PfLds {
     const int16_t* bs;   // N x N, bs[i*N + j] = index-map entry b(i, j)
     const cplx<R>* fs;   // rows x 4: fs[r*4 + c]
     int N, rows;
-    cplx<R>* X;          // this wave's exchange / accumulator scratch
-    cplx<double>* Xd;    // the same region as N x N complex double
+    // this wave's scratch, by use
+    cplx<R>* X;          // derivative sums
+    double* Xr;          // N x (N + 1): one part of a matrix, entry (i, j) at j (N + 1) + i
+    cplx<double>* Xd;    // N x N (scratch with room for it)
     cplx<R>* D;          // 8 x 32
-    cplx<R>* G;          // 16 x 16
-    int* F;              // 16 ints: the flip list of the current ratio
+    cplx<R>* G;          // 16 x 16, after D
+    int* F;              // 16 ints after G: the flip list of the current ratio
 };
 
 __device__ inline int bit2(const uint64_t* st, int i) { return (int)((st[i >> 6] >> (i & 63)) & 1); }
@@ -74,9 +87,109 @@ __device__ inline cplx<R> cdiv(cplx<R> a, cplx<R> b) {
     return {(a.re * b.re + a.im * b.im) * d, (a.im * b.re - a.re * b.im) * d};
 }
 
+// a b with the roundings of each part spelled out: an incremental inverse in
+// FP32 is sensitive to the last bit (chains leave each other within an epoch),
+// so the products here are not left to the compiler's choice of which product
+// an FMA takes, and the order of their factors matters: pmul(a, b) and pmul(b,
+// a) differ in the imaginary part
+template <typename R>
+__device__ inline cplx<R> pmul(cplx<R> a, cplx<R> b) {
+    if constexpr (sizeof(R) == 4)
+        return {__builtin_fmaf(a.re, b.re, -(a.im * b.im)), __builtin_fmaf(a.im, b.re, a.re * b.im)};
+    else return {__builtin_fma(a.re, b.re, -(a.im * b.im)), __builtin_fma(a.im, b.re, a.re * b.im)};
+}
+
+// -a b; the real part rounds the product of the real parts
+template <typename R>
+__device__ inline cplx<R> pmuln(cplx<R> a, cplx<R> b) {
+    if constexpr (sizeof(R) == 4)
+        return {__builtin_fmaf(a.im, b.im, -(a.re * b.re)), -__builtin_fmaf(a.im, b.re, a.re * b.im)};
+    else return {__builtin_fma(a.im, b.im, -(a.re * b.re)), -__builtin_fma(a.im, b.re, a.re * b.im)};
+}
+
+// 1 / a
+template <typename R>
+__device__ inline cplx<R> pinv(cplx<R> a) {
+    R d;
+    if constexpr (sizeof(R) == 4) d = 1 / __builtin_fmaf(a.re, a.re, a.im * a.im);
+    else d = 1 / __builtin_fma(a.re, a.re, a.im * a.im);
+    return {a.re * d, -a.im * d};
+}
+
 template <typename R>
 __device__ inline cplx<R> shfl_c(cplx<R> v, int src) {
     return {__shfl(v.re, src), __shfl(v.im, src)};
+}
+
+// both halves of a value's 16-lane row pairs / 32-lane halves: (even row or
+// low half, odd row or high half), the same in both partners
+template <typename T>
+struct Two {
+    T lo, hi;
+};
+__device__ inline Two<uint32_t> swap16(uint32_t v) {
+    const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    return {r[0], r[1]};
+}
+__device__ inline Two<uint32_t> swap32(uint32_t v) {
+    const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return {r[0], r[1]};
+}
+template <bool W32>
+__device__ inline Two<float> swp(float v) {
+    const Two<uint32_t> r = W32 ? swap32(__float_as_uint(v)) : swap16(__float_as_uint(v));
+    return {__uint_as_float(r.lo), __uint_as_float(r.hi)};
+}
+template <bool W32>
+__device__ inline Two<double> swp(double v) {
+    const Two<uint32_t> a = W32 ? swap32((uint32_t)__double2loint(v)) : swap16((uint32_t)__double2loint(v));
+    const Two<uint32_t> b = W32 ? swap32((uint32_t)__double2hiint(v)) : swap16((uint32_t)__double2hiint(v));
+    return {__hiloint2double((int)b.lo, (int)a.lo), __hiloint2double((int)b.hi, (int)a.hi)};
+}
+template <bool W32, typename R>
+__device__ inline Two<cplx<R>> swp(cplx<R> v) {
+    const Two<R> a = swp<W32>(v.re), b = swp<W32>(v.im);
+    return {{a.lo, b.lo}, {a.hi, b.hi}};
+}
+// lane n of each 16-lane row to the whole row
+template <int n>
+__device__ inline float row_bcast(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + n, 0xF, 0xF, false));
+}
+template <int n>
+__device__ inline double row_bcast(double v) {
+    return __longlong_as_double(__builtin_amdgcn_update_dpp(0LL, __double_as_longlong(v), 0x150 + n, 0xF, 0xF, false));
+}
+template <int n, typename R>
+__device__ inline cplx<R> row_bcast(cplx<R> v) {
+    return {row_bcast<n>(v.re), row_bcast<n>(v.im)};
+}
+// f(integral_constant<I>) .. f(integral_constant<n - 1>)
+template <int I, int n, typename F>
+__device__ __attribute__((always_inline)) inline void unroll_n(F&& f) {
+    if constexpr (I < n) {
+        f(std::integral_constant<int, I>{});
+        unroll_n<I + 1, n>(f);
+    }
+}
+// lane src (wave-uniform) of v as a wave-uniform value
+__device__ inline float lane_of(float v, int src) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), src));
+}
+__device__ inline double lane_of(double v, int src) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), src),
+                            __builtin_amdgcn_readlane(__double2loint(v), src));
+}
+template <typename R>
+__device__ inline cplx<R> lane_of(cplx<R> v, int src) {
+    return {lane_of(v.re, src), lane_of(v.im, src)};
+}
+// group_csum<32> with the last step by v_permlane16_swap: the same sums
+template <typename R>
+__device__ inline cplx<R> csum32(cplx<R> v) {
+    v = group_csum<16>(v);
+    const Two<cplx<R>> t = swp<false>(v);
+    return t.lo + t.hi;
 }
 
 // wave argmax of key over lanes (ties: smaller lane); returns the lane
@@ -106,83 +219,101 @@ __device__ inline void pf_build(const PfLds<R>& l, const uint64_t* st, int lane)
     wave_sync();
 }
 
-// Gauss-Jordan inverse of Xd in place (FP64) with partial pivoting (row swaps,
-// columns unscrambled at the end); returns false if singular
-template <typename R>
-__device__ inline bool pf_gj(const PfLds<R>& l, int lane, int& ipiv_lane) {
-    const int N = l.N;
-    cplx<double>* X = l.Xd;
-    bool ok = true;
-    for (int c = 0; c < N; c++) {
-        double key = -1;
-        if (lane < N && lane >= c) {
-            cplx<double> x = X[c * N + lane];
-            key = (double)x.re * x.re + (double)x.im * x.im;
-        }
-        int p = wave_argmax(key, lane);
-        if (lane == c) ipiv_lane = p;
-        if (p != c) {
-            if (lane < N) {
-                cplx<double> a = X[lane * N + p], b = X[lane * N + c];
-                X[lane * N + p] = b;
-                X[lane * N + c] = a;
-            }
-            wave_sync();
-        }
-        cplx<double> piv = X[c * N + c];
-        if (piv.re == 0 && piv.im == 0) ok = false;
-        cplx<double> inv = cdiv(cplx<double>{1, 0}, piv);
-        // row c: X(c, c) := 1, then row c *= 1 / piv
-        if (lane < N) {
-            cplx<double> t = lane == c ? cplx<double>{1, 0} : X[lane * N + c];
-            X[lane * N + c] = t * inv;
-        }
-        wave_sync();
-        // other rows: X(r, j) -= X(r, c) X(c, j), with X(r, c) := 0 first;
-        // column c is snapshotted into the G area so no lane reads an
-        // entry another lane has already rewritten (row c is not written)
-        cplx<double>* col = reinterpret_cast<cplx<double>*>(l.G);
-        if (lane < N) col[lane] = X[c * N + lane];
-        wave_sync();
-        for (int e = lane; e < N * N; e += 64) {
-            int r = e % N, j = e / N;
-            if (r == c) continue;
-            cplx<double> x = j == c ? cplx<double>{0, 0} : X[e];
-            X[e] = x - col[r] * X[j * N + c];
-        }
-        wave_sync();
-    }
-    // unscramble: columns swapped in reverse pivot order
-    for (int c = N - 1; c >= 0; c--) {
-        int p = __shfl(ipiv_lane, c);
-        if (p != c) {
-            if (lane < N) {
-                cplx<double> a = X[p * N + lane], b = X[c * N + lane];
-                X[p * N + lane] = b;
-                X[c * N + lane] = a;
-            }
-            wave_sync();
-        }
-    }
-    return ok;
-}
-
-// fresh FP64 inverse of A(sigma), antisymmetrised (pfaffian.cpp:284-297), into v
+// fresh FP64 inverse of A(sigma), antisymmetrised (pfaffian.cpp:284-297), into
+// v: Gauss-Jordan with partial pivoting in registers, lane l holding row i = l
+// & 31, columns 16h .. 16h + 15.  Rows stay in their lanes; pos is the row's
+// place under the row swaps (ties between pivots go to the smaller place), the
+// columns are unscrambled and the matrix transposed through LDS at the end, one
+// part at a time.  Returns false if singular.
 template <typename R>
 __device__ inline bool pf_fresh(const PfLds<R>& l, const uint64_t* st, int lane, cplx<R> (&v)[16]) {
-    pf_build(l, st, lane);
-    int ip = 0;
-    bool ok = pf_gj(l, lane, ip);
-    const int i = lane & 31, h = lane >> 5, N = l.N;
+    const int N = l.N, i = lane & 31, h = lane >> 5;
+    cplx<double> x[16];
+    const int si = i < N ? bit2(st, i) : 0;
 #pragma unroll
     for (int q = 0; q < 16; q++) {
-        int j = 16 * h + q;
-        cplx<R> r{0, 0};
+        const int j = 16 * h + q;
+        x[q] = {0, 0};
         if (i < N && j < N) {
-            cplx<double> a = l.Xd[j * N + i], b = l.Xd[i * N + j];
-            r = {(R)(0.5 * (a.re - b.re)), (R)(0.5 * (a.im - b.im))};
+            const cplx<R> a = pf_a(l, i, j, si, bit2(st, j));
+            x[q] = {(double)a.re, (double)a.im};
         }
-        v[q] = r;
+    }
+    bool ok = true;
+    int pos = i, ip = i;  // ip: lane c holds the place swapped with place c
+    for (int hc = 0; hc < 2; hc++)
+        unroll_n<0, 16>([&](auto qc) __attribute__((always_inline)) {
+            constexpr int q0 = decltype(qc)::value;
+            const int c = 16 * hc + q0;
+            if (c >= N) return;
+            // column c of the lane's row, in both halves
+            const Two<cplx<double>> t = swp<true>(x[q0]);
+            const cplx<double> col = hc ? t.hi : t.lo;
+            // pivot: the largest |X(row, c)|^2 at places >= c, the smallest place among equals
+            double key = -1;
+            if (i < N && pos >= c) key = col.re * col.re + col.im * col.im;
+            double best = key;
+            best = fmax(best, partner<1>(best));
+            best = fmax(best, partner<2>(best));
+            best = fmax(best, partner<4>(best));
+            best = fmax(best, partner<8>(best));
+            {
+                const Two<double> m = swp<false>(best);
+                best = fmax(m.lo, m.hi);
+            }
+            int p = i < N && pos >= c && (key == best || !(best == best)) ? pos : 64;
+            p = min(p, partner<1>(p));
+            p = min(p, partner<2>(p));
+            p = min(p, partner<4>(p));
+            p = min(p, partner<8>(p));
+            {
+                const Two<uint32_t> m = swap16((uint32_t)p);
+                p = min((int)m.lo, (int)m.hi);
+            }
+            p = __builtin_amdgcn_readfirstlane(p < 64 ? p : c);
+            const int prow = __builtin_ctzll(__ballot(pos == p));  // lane of the pivot row (low half)
+            if (lane == c) ip = p;
+            if (pos == c) pos = p;
+            else if (i == prow) pos = c;
+            const cplx<double> piv = lane_of(col, prow);
+            if (piv.re == 0 && piv.im == 0) ok = false;
+            const cplx<double> inv = cdiv(cplx<double>{1, 0}, piv);
+            // the pivot row (with 1 at column c) times 1 / piv, then subtracted
+            // from every other row (with 0 at column c)
+#pragma unroll
+            for (int q = 0; q < 16; q++) {
+                const cplx<double> r0 = lane_of(x[q], prow), r1 = lane_of(x[q], prow + 32);
+                cplx<double> row = h ? r1 : r0;
+                const bool at = q == q0 && h == hc;
+                if (at) row = {1, 0};
+                row = row * inv;
+                const cplx<double> xq = at ? cplx<double>{0, 0} : x[q];
+                x[q] = i == prow ? row : xq - col * row;
+            }
+        });
+    // where column k (lane k) ends: swaps in reverse pivot order
+    int loc = i;
+    for (int c = N - 1; c >= 0; c--) {
+        const int p = __builtin_amdgcn_readlane(ip, c);
+        loc = loc == p ? c : loc == c ? p : loc;
+    }
+#pragma unroll
+    for (int part = 0; part < 2; part++) {
+        wave_sync();
+#pragma unroll
+        for (int q = 0; q < 16; q++) {
+            const int c0 = __builtin_amdgcn_readlane(loc, q), c1 = __builtin_amdgcn_readlane(loc, 16 + q);
+            if (i < N && 16 * h + q < N) l.Xr[(h ? c1 : c0) * (N + 1) + pos] = part ? x[q].im : x[q].re;
+        }
+        wave_sync();
+#pragma unroll
+        for (int q = 0; q < 16; q++) {
+            const int j = 16 * h + q;
+            R r = 0;
+            if (i < N && j < N) r = (R)(0.5 * (l.Xr[j * (N + 1) + i] - l.Xr[i * (N + 1) + j]));
+            if (part) v[q].im = r;
+            else v[q].re = r;
+        }
     }
     wave_sync();
     return ok;
@@ -278,24 +409,113 @@ __device__ inline cplx<R> small_pf(cplx<R>* G, int m, int lane) {
 template <typename R, bool KEEP>
 struct PfProp {
     cplx<R> ib[KEEP ? 4 : 1];
+    cplx<R> g[KEEP ? 6 : 1];  // upper triangle 01, 02, 03, 12, 13, 23 of Cinv' (m = 1: 01)
     int m;
 };
 
+// v[f & 15] of the half f >> 4, in both halves (f wave-uniform)
+template <typename R>
+__device__ inline cplx<R> pf_column(const cplx<R> (&v)[16], int f) {
+    cplx<R> sel = v[0];
+#pragma unroll
+    for (int q = 1; q < 16; q++)
+        if (q == (f & 15)) sel = v[q];
+    const Two<cplx<R>> t = swp<true>(sel);
+    return (f >> 4) ? t.hi : t.lo;
+}
+// value of lane (i, h) -> value of index 16 h + (lane & 15)
+template <typename R>
+__device__ inline cplx<R> to_half(cplx<R> v, int h) {
+    const Two<cplx<R>> t = swp<false>(v);
+    return h ? t.hi : t.lo;
+}
+
+// pf_ratio for one or two flipped sites f0 (, f1; -1: one), wave-uniform: the
+// entries of G = B^T inv B that Cinv' reads, each formed as pf_ratio forms it
+template <typename R, bool KEEP>
+__device__ inline cplx<R> pf_ratio2(const PfLds<R>& l, const cplx<R> (&v)[16], const uint64_t* st, int f0, int f1,
+                                    int lane, PfProp<R, KEEP>& pp) {
+    const int N = l.N, i = lane & 31, h = lane >> 5;
+    const bool two = f1 >= 0;
+    const int s0 = bit2(st, f0), s1 = two ? bit2(st, f1) : 0;
+    const int si = i < N ? bit2(st, i) : 0, sn = si ^ (i == f0 || i == f1);
+    // Delta-a rows a(i, f; flipped) - a(i, f)
+    cplx<R> d0{0, 0}, d1{0, 0};
+    if (i < N && i != f0) d0 = pf_a(l, i, f0, sn, s0 ^ 1) - pf_a(l, i, f0, si, s0);
+    if (two && i < N && i != f1) d1 = pf_a(l, i, f1, sn, s1 ^ 1) - pf_a(l, i, f1, si, s1);
+    // columns inv Delta-a and inv e_f
+    auto mv = [&](cplx<R> d) __attribute__((always_inline)) {
+        const cplx<R> e = to_half(d, h);
+        cplx<R> s{0, 0};
+        unroll_n<0, 16>([&](auto qc) __attribute__((always_inline)) {
+            constexpr int q = decltype(qc)::value;
+            s = s + pmul(v[q], row_bcast<q>(e));
+        });
+        const Two<cplx<R>> t = swp<true>(s);
+        return t.lo + t.hi;
+    };
+    auto half = [](cplx<R> a, cplx<R> b) { return cplx<R>{(R)0.5 * (a.re - b.re), (R)0.5 * (a.im - b.im)}; };
+    pp.m = two ? 2 : 1;
+    const cplx<R> c0 = mv(d0);
+    if (!two) {
+        const cplx<R> e0 = pf_column(v, f0);
+        cplx<R> g01 = half(csum32(pmul(e0, d0)), lane_of(c0, f0));
+        g01.re -= 1;
+        if constexpr (KEEP) {
+            pp.ib[0] = c0;
+            pp.ib[1] = e0;
+            pp.ib[2] = pp.ib[3] = {0, 0};
+            pp.g[0] = g01;
+        }
+        return {-g01.re, -g01.im};
+    }
+    const cplx<R> c1 = mv(d1);
+    const cplx<R> e0 = pf_column(v, f0), e1 = pf_column(v, f1);
+    cplx<R> g01 = half(csum32(pmul(c1, d0)), csum32(pmul(c0, d1)));
+    cplx<R> g02 = half(csum32(pmul(e0, d0)), lane_of(c0, f0)), g03 = half(csum32(pmul(e1, d0)), lane_of(c0, f1));
+    cplx<R> g12 = half(csum32(pmul(e0, d1)), lane_of(c1, f0)), g13 = half(csum32(pmul(e1, d1)), lane_of(c1, f1));
+    const cplx<R> g23 = half(lane_of(e1, f0), lane_of(e0, f1));
+    g02.re -= 1;
+    g13.re -= 1;
+    // pair entry Cinv0(1, 0) = a(f1, f0) - a(f1, f0; both flipped)
+    g01 = g01 - (pf_a(l, f1, f0, s1, s0) - pf_a(l, f1, f0, s1 ^ 1, s0 ^ 1));
+    if constexpr (KEEP) {
+        pp.ib[0] = c0;
+        pp.ib[1] = c1;
+        pp.ib[2] = e0;
+        pp.ib[3] = e1;
+        pp.g[0] = g01;
+        pp.g[1] = g02;
+        pp.g[2] = g03;
+        pp.g[3] = g12;
+        pp.g[4] = g13;
+        pp.g[5] = g23;
+    }
+    const cplx<R> pf = pmul(g01, g23) - pmul(g02, g13) + pmul(g03, g12);
+    return {-pf.re, -pf.im};
+}
+
 // Pf(A(sigma')) / Pf(A(sigma)) for sigma' = sigma with the sites fl[i]
 // (bit i of mask set, i < 8) flipped, in increasing i (uniform over the
-// wave); leaves Cinv' in G (row-major, stride 16).  KEEP: at most the
-// first two slots are used (single and bond flips) and the columns of
-// inv B of this lane's row are kept for pf_accept.
-template <typename R, bool KEEP>
+// wave).  One or two sites by pf_ratio2, more through D and G in LDS.
+template <typename R>
 __device__ inline cplx<R> pf_ratio(const PfLds<R>& l, const cplx<R> (&v)[16], const uint64_t* st, const int* fl,
-                                   int mask, int lane, PfProp<R, KEEP>& pp) {
-    constexpr int NS = KEEP ? 2 : 8;  // flip slots
+                                   int mask, int lane) {
+    constexpr int NS = 8;  // flip slots
     const int N = l.N, i = lane & 31, h = lane >> 5;
     const int m = __builtin_popcount(mask);
-    pp.m = m;
-    if constexpr (KEEP)
+    if (m <= 2) {
+        int f0 = -1, f1 = -1;
 #pragma unroll
-        for (int u = 0; u < 4; u++) pp.ib[u] = {0, 0};
+        for (int t = 0; t < NS; t++)
+            if ((mask >> t) & 1) {
+                if (f0 < 0) f0 = fl[t];
+                else f1 = fl[t];
+            }
+        PfProp<R, false> pp;
+        return pf_ratio2<R, false>(l, v, st, __builtin_amdgcn_readfirstlane(f0), __builtin_amdgcn_readfirstlane(f1),
+                                   lane, pp);
+    }
     // compacted flip list (uniform) -> F
     if (lane == 0) {
         int k = 0;
@@ -330,11 +550,6 @@ __device__ inline cplx<R> pf_ratio(const PfLds<R>& l, const cplx<R> (&v)[16], co
                 if (q == (f & 15)) sel = v[q];
             cplx<R> oth{partner<32>(sel.re), partner<32>(sel.im)};
             col = (f >> 4) == h ? sel : oth;
-        }
-        if constexpr (KEEP) {
-#pragma unroll
-            for (int u = 0; u < 4; u++)
-                if (u == b) pp.ib[u] = col;
         }
         for (int a = 0; a < m; a++) {
             // rows a < m: sum_i Delta-a_a(i) col(i); rows m + a: col(f_a)
@@ -388,58 +603,69 @@ __device__ inline cplx<R> pf_ratio(const PfLds<R>& l, const cplx<R> (&v)[16], co
     return neg ? cplx<R>{-pf.re, -pf.im} : pf;
 }
 
-// accept the flip set of the last pf_ratio<R, true> (m <= 2), whose Cinv'
-// is in G.  C = antisym(Cinv'^-1 / 2) = Cinv'^-1 for the skew Cinv', by
+// accept the flip set of the last pf_ratio2<R, true>, whose Cinv' is in
+// pp.g.  C = antisym(Cinv'^-1 / 2) = Cinv'^-1 for the skew Cinv', by
 // the closed forms of the 2 x 2 and 4 x 4 skew inverses:
 //   [[0, x], [-x, 0]]^-1 = [[0, -1/x], [1/x, 0]],
 //   A^-1 = (1/Pf A) [[0, -a23, a13, -a12], [a23, 0, -a03, a02],
 //                    [-a13, a03, 0, -a01], [a12, -a02, a01, 0]].
 template <typename R>
 __device__ inline void pf_accept(const PfLds<R>& l, cplx<R> (&v)[16], const PfProp<R, true>& pp, int lane) {
-    const int m = pp.m, n = 2 * m, i = lane & 31, h = lane >> 5;
+    const int m = pp.m, n = 2 * m, h = lane >> 5;
     // upper triangle c01, c02, c03, c12, c13, c23 of C
     cplx<R> c01, c02{0, 0}, c03{0, 0}, c12{0, 0}, c13{0, 0}, c23{0, 0};
     if (m == 1) {
-        c01 = cdiv(cplx<R>{-1, 0}, l.G[1]);
+        const cplx<R> ip = pinv(pp.g[0]);
+        c01 = {-ip.re, -ip.im};
     } else {
-        cplx<R> a01 = l.G[1], a02 = l.G[2], a03 = l.G[3], a12 = l.G[16 + 2], a13 = l.G[16 + 3],
-                a23 = l.G[32 + 3];
-        cplx<R> ip = cdiv(cplx<R>{1, 0}, a01 * a23 - a02 * a13 + a03 * a12);
-        c01 = cplx<R>{-a23.re, -a23.im} * ip;
-        c02 = a13 * ip;
-        c03 = cplx<R>{-a12.re, -a12.im} * ip;
-        c12 = cplx<R>{-a03.re, -a03.im} * ip;
-        c13 = a02 * ip;
-        c23 = cplx<R>{-a01.re, -a01.im} * ip;
+        cplx<R> a01 = pp.g[0], a02 = pp.g[1], a03 = pp.g[2], a12 = pp.g[3], a13 = pp.g[4], a23 = pp.g[5];
+        const cplx<R> ip = pinv(pmul(a01, a23) - pmul(a02, a13) + pmul(a03, a12));
+        // times 1 / Pf; the products' rounding differs between the precisions
+        auto by = [&](cplx<R> a) { return sizeof(R) == 4 ? pmul(ip, a) : pmul(a, ip); };
+        auto byn = [&](cplx<R> a) { return cplx<R>{pmuln(a, ip).re, sizeof(R) == 4 ? pmuln(a, ip).im : -pmul(ip, a).im}; };
+        c01 = byn(a23);
+        c02 = by(a13);
+        c03 = byn(a12);
+        c12 = byn(a03);
+        c13 = by(a02);
+        c23 = byn(a01);
     }
     auto neg = [](cplx<R> x) { return cplx<R>{-x.re, -x.im}; };
     // t1 = (inv B) C for this lane's row
     cplx<R> t1[4];
-    t1[0] = neg(pp.ib[1] * c01) - pp.ib[2] * c02 - pp.ib[3] * c03;
-    t1[1] = pp.ib[0] * c01 - pp.ib[2] * c12 - pp.ib[3] * c13;
-    t1[2] = pp.ib[0] * c02 + pp.ib[1] * c12 - pp.ib[3] * c23;
-    t1[3] = pp.ib[0] * c03 + pp.ib[1] * c13 + pp.ib[2] * c23;
-    // exchange rows of inv B and t1 through X: X[b*32 + i], X[(4 + b)*32 + i]
-    if (h == 0)
+    const cplx<R>(&ib)[4] = pp.ib;
+    t1[0] = neg(pmul(ib[1], c01)) - pmul(c02, ib[2]) - pmul(c03, ib[3]);
+    t1[1] = pmul(ib[0], c01) - pmul(c12, ib[2]) - pmul(c13, ib[3]);
+    t1[2] = pmul(c02, ib[0]) + pmul(c12, ib[1]) - pmul(c23, ib[3]);
+    t1[3] = pmul(c03, ib[0]) + pmul(c13, ib[1]) + pmul(c23, ib[2]);
+    // inv(i, j) += (1/2) sum_b [t1(i, b) invB(j, b) - t1(j, b) invB(i, b)], the
+    // rows j = 16 h + q of inv B and t1 by row broadcasts
+    cplx<R> eb[4], et[4];
 #pragma unroll
-        for (int b = 0; b < 4; b++) {
-            if (b < n) {
-                l.X[b * 32 + i] = pp.ib[b];
-                l.X[(4 + b) * 32 + i] = t1[b];
-            }
+    for (int b = 0; b < 4; b++)
+        if (b < n) {
+            eb[b] = to_half(pp.ib[b], h);
+            et[b] = to_half(t1[b], h);
         }
-    wave_sync();
-    // inv(i, j) += (1/2) sum_b [t1(i, b) invB(j, b) - t1(j, b) invB(i, b)]
+    auto update = [&](auto nc) __attribute__((always_inline)) {
+        constexpr int nb = decltype(nc)::value;
+        unroll_n<0, 16>([&](auto qc) __attribute__((always_inline)) {
+            constexpr int q = decltype(qc)::value;
+            cplx<R> s{0, 0};
 #pragma unroll
-    for (int q = 0; q < 16; q++) {
-        int j = 16 * h + q;
-        cplx<R> s{0, 0};
-#pragma unroll
-        for (int b = 0; b < 4; b++)
-            if (b < n) s = s + t1[b] * l.X[b * 32 + j] - l.X[(4 + b) * 32 + j] * pp.ib[b];
-        v[q] = v[q] + cplx<R>{(R)0.5 * s.re, (R)0.5 * s.im};
-    }
-    wave_sync();
+            for (int b = 0; b < nb; b++) {
+                const cplx<R> tj = row_bcast<q>(et[b]);
+                s = s + pmul(t1[b], row_bcast<q>(eb[b]));
+                if (b < 3) {
+                    const cplx<R> u = pmuln(ib[b], tj);
+                    s = {s.re + u.re, s.im + u.im};
+                } else s = s - pmul(ib[b], tj);
+            }
+            v[q] = v[q] + cplx<R>{(R)0.5 * s.re, (R)0.5 * s.im};
+        });
+    };
+    if (m == 1) update(std::integral_constant<int, 2>{});
+    else update(std::integral_constant<int, 4>{});
 }
 
 // d ln Pf / d fs (pfaffian.cpp:399-415) summed into out[n_pf] (this wave's
@@ -448,6 +674,7 @@ template <typename R>
 __device__ inline void pf_derivative(const PfLds<R>& l, const cplx<R> (&v)[16], const uint64_t* st, int lane,
                                      cplx<R>* out) {
     const int N = l.N, i = lane & 31, h = lane >> 5, npf = 4 * l.rows;
+    wave_sync();
     for (int e = lane; e < npf; e += 64) l.X[e] = {0, 0};
     wave_sync();
     if (i < N) {

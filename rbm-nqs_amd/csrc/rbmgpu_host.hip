@@ -209,9 +209,9 @@ size_t rsize(const rbmgpu_ctx* c) { return c->prec == RBMGPU_FP32 ? 4 : 8; }
 
 // LDS staging: everything if it fits, else drop the local-operator tables,
 // then W (both are then read from memory)
-Dims dims(const rbmgpu_ctx* c, int block = 256) {
+Dims dims(const rbmgpu_ctx* c, int block = 256, int pf_full = 0) {
     Dims d{c->N, c->H, c->na, c->nsymm, c->nvb, c->nw, 1, 1, (int)c->pb.size() / 2, c->n_terms, c->n_rowptr,
-           c->n_ent, c->pf_rows, block / 64};
+           c->n_ent, c->pf_rows, block / 64, pf_full};
     auto fits = [&] {
         return (c->prec == RBMGPU_FP32 ? lds_bytes<float>(d) : lds_bytes<double>(d)) <= c->lds_limit;
     };
@@ -321,14 +321,16 @@ bool shape_fits(const rbmgpu_ctx* c, Shape s) {
 }
 
 // block size: 256 threads unless that leaves fewer than two blocks per CU;
-// with the Pfaffian also small enough for its per-wave LDS scratch
-int pick_block(const rbmgpu_ctx* c, int L, int64_t groups) {
-    int b = 256;
-    while (b > 64 && groups * L / b < 2 * c->n_cu) b /= 2;
+// with the Pfaffian in FP32 up to kPfBlock, as long as every CU gets a block,
+// and small enough for its per-wave LDS scratch
+int pick_block(const rbmgpu_ctx* c, int L, int64_t groups, int pf_full = 0) {
+    const bool pf = c->pf_rows && c->prec == RBMGPU_FP32;
+    int b = pf ? kPfBlock : 256;
+    while (b > 64 && groups * L / b < (pf ? 1 : 2) * c->n_cu) b /= 2;
     b = std::max(b, L);
     if (c->pf_rows)
-        while (b > 64 && (c->prec == RBMGPU_FP32 ? lds_bytes<float>(dims(c, b)) : lds_bytes<double>(dims(c, b))) >
-                             c->lds_limit)
+        while (b > 64 && (c->prec == RBMGPU_FP32 ? lds_bytes<float>(dims(c, b, pf_full))
+                                                 : lds_bytes<double>(dims(c, b, pf_full))) > c->lds_limit)
             b /= 2;
     return b;
 }
@@ -1653,8 +1655,9 @@ int run_eval(rbmgpu_ctx* c, const uint64_t* d_states, int64_t n, double* logpsi,
             }
         }
     }
-    int block = pick_block(c, s.L, n);
-    a.d = dims(c, block);
+    const int full = c->pf_rows && logpsi ? 1 : 0;
+    const int block = std::min(256, pick_block(c, s.L, n, full));
+    a.d = dims(c, block, full);
     HIPCK(launch_eval<R>(a, s, block, c->stream));
     return 0;
 }
