@@ -243,6 +243,18 @@ __device__ inline T group_sum(T v) {
         return v;
     }
 }
+// mantissa in [0.5, 1) and exponent (0, inf and NaN: themselves and 0)
+__device__ inline double frexp_m(double x) { return __builtin_amdgcn_frexp_mant(x); }
+__device__ inline int frexp_e(double x) { return __builtin_amdgcn_frexp_exp(x); }
+// product of the group's m 2^e, m as frexp_m gives it
+template <int L, int O = 1>
+__device__ inline void group_prod(double& m, int& e) {
+    if constexpr (O < L) {
+        m *= partner<O>(m);
+        e += partner<O>(e);
+        group_prod<L, 2 * O>(m, e);
+    }
+}
 template <int L, int O = 1>
 __device__ inline float group_max(float v) {
     if constexpr (O < L) {

@@ -110,15 +110,15 @@ template <typename R, int L, int K>
 struct Units {
     int a[K], s[K];  // alpha and symmetry index per unit, a < 0: padding
     cplx<R> th[K], tn[K];
-    // FP32 (K <= 4; more units would cost occupancy): cosh and
+    // K <= 4 in FP32, K <= 2 in FP64 (more units would cost occupancy): cosh and
     // sinh of the last ratio12 flip set's delta per unit and the unit's
     // ratio factor cosh(theta + delta) / cosh(theta), kept for accept12's
     // tanh update
-    static constexpr bool kMob = sizeof(R) == 4 && K <= 4;
-    // FP32 with more units per lane: the same Mobius step, its cosh / sinh
+    static constexpr bool kMob = sizeof(R) == 4 ? K <= 4 : K <= 2;
+    // more units per lane: the same Mobius step, its cosh / sinh
     // factors reloaded from the tables at the (less frequent) accepted move
     // instead of kept in registers from the ratio
-    static constexpr bool kMobR = sizeof(R) == 4 && !kMob;
+    static constexpr bool kMobR = !kMob;
     cplx<R> kc[kMob ? K : 1], ks[kMob ? K : 1], kr[kMob ? K : 1];
     // K <= 2, L <= 32 (the Pfaffian shapes have L = 64 and no registers to
     // spare): W entries of the last ratio12 flip set, loaded with its C
@@ -241,14 +241,12 @@ struct Units {
             if (sizeof(R) == 4 && (u & 3) == 3) renorm(p, pe);
         }
     }
-    // FP32 (kMob) after a sweep: tanh from theta again (the accepted moves
-    // update tanh incrementally, see accept12_w)
+    // after a sweep: tanh from theta again (the accepted moves update tanh
+    // incrementally, see accept12_w)
     __device__ void resync() {
-        if constexpr (kMob || kMobR) {
 #pragma unroll
-            for (int u = 0; u < K; u++)
-                if (a[u] >= 0) tn[u] = ctanh(th[u]);
-        }
+        for (int u = 0; u < K; u++)
+            if (a[u] >= 0) tn[u] = ctanh(th[u]);
     }
     // generic flip set: sites fl[i] for i < 8 with bit i of mask set
     __device__ void ratio_mask(const Dims& d, const Lds<R>& l, const int* fl, const R* sg, int mask,
@@ -295,13 +293,14 @@ struct Units {
         else
             accept12_w(d, l, l.Wg, f0, s0, f1, s1);
     }
-    // FP64 recomputes tanh(theta) (the chains follow the oracle's state for
-    // state); FP32 (kMob) updates it from the ratio12 of the same flip set:
+    // tanh is updated from the ratio12 of the same flip set:
     // tanh(theta + delta) = (t cosh delta + sinh delta) / (cosh delta +
     // t sinh delta), whose denominator is the unit's ratio factor (a move
     // is accepted with probability |prod of factors|^2, so a vanishing
     // factor is almost never divided by); resync() restores tanh(theta)
-    // after every sweep, so rounding builds up over one sweep at most
+    // after every sweep, so rounding builds up over one sweep at most, and
+    // what is written of a kept sample is tanh(theta) itself.  theta moves by
+    // the same sums as ever
     __device__ void accept12_w(const Dims& d, const Lds<R>& l, const cplx<R>* W, int f0, R s0, int f1, R s1) {
         if constexpr (!kPreW) {  // unit by unit
 #pragma unroll
@@ -329,7 +328,7 @@ struct Units {
                 if constexpr (kMobR) {
                     // tanh(theta + delta) = (t cosh delta + sinh delta) / (cosh delta + t sinh delta)
                     const cplx<R> num = tn[u] * ch + sh, r = ch + tn[u] * sh;
-                    const R inv = __builtin_amdgcn_rcpf(r.re * r.re + r.im * r.im);
+                    const R inv = rcp(r.re * r.re + r.im * r.im);
                     tn[u] = {(num.re * r.re + num.im * r.im) * inv, (num.im * r.re - num.re * r.im) * inv};
                 } else {
                     update_tanh(u);
@@ -346,14 +345,12 @@ struct Units {
         }
     }
     __device__ void update_tanh(int u) {
-        if constexpr (kMob) {
-            const cplx<R> num = tn[u] * kc[u] + ks[u], r = kr[u];
-            const R inv = __builtin_amdgcn_rcpf(r.re * r.re + r.im * r.im);
-            tn[u] = {(num.re * r.re + num.im * r.im) * inv, (num.im * r.re - num.re * r.im) * inv};
-        } else {
-            tn[u] = ctanh(th[u]);
-        }
+        const cplx<R> num = tn[u] * kc[u] + ks[u], r = kr[u];
+        const R inv = rcp(r.re * r.re + r.im * r.im);
+        tn[u] = {(num.re * r.re + num.im * r.im) * inv, (num.im * r.re - num.re * r.im) * inv};
     }
+    static __device__ float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
+    static __device__ double rcp(double x) { return 1 / x; }
 };
 
 // psi(sigma')/psi(sigma) for the sites of a term selected by mask: the
@@ -651,6 +648,10 @@ __device__ inline void eval_obs(const Dims& d, const Lds<R>& l, const Units<R, L
 // bond_flips both ends of a random non-z bond are flipped (taking two
 // slots), else one uniform site; accept if u < |psi'/psi|^2.  At kept
 // steps the local observables and tanh(theta) of the sample are written.
+// A chain is one dependent sequence of proposals, so with few chains the sampler
+// is bound by a proposal's latency: in FP64 the decision takes no logarithm and
+// the accepted move no exponential or sine (toric 4x4 symmetric, 64 chains, 450
+// sweeps: 13.9 -> 9.6 ms; basic, 4096 chains x 164 sweeps: 15.5 -> 12.3 ms).
 // With the Pfaffian factor in FP32 up to 8 chains share a block's tables: its
 // LDS lets one block per CU run (Kitaev 4x4), as two wavefronts per SIMD of 256
 // registers; in FP64 one of 512 registers.
@@ -716,8 +717,15 @@ __global__ void __launch_bounds__(PF && sizeof(R) == 4 ? kPfBlock : 256) k_sampl
                 sw0 = sw & ~(L - 1);
                 draw(step, sw0);
             }
-            int code = __shfl(pcode, sw - sw0, L);
-            R uu = __shfl(pu, sw - sw0, L);
+            int code;
+            R uu;
+            if constexpr (L == 64 && sizeof(R) == 8) {  // one chain per wavefront
+                code = __builtin_amdgcn_readlane(pcode, sw - sw0);
+                uu = lane_of(pu, sw - sw0);
+            } else {
+                code = __shfl(pcode, sw - sw0, L);
+                uu = __shfl(pu, sw - sw0, L);
+            }
             int f0 = code & 0xFF, f1 = (code >> 8) - 1;
             if (f1 >= 0) sw++;
             prop++;
@@ -726,19 +734,42 @@ __global__ void __launch_bounds__(PF && sizeof(R) == 4 ? kPfBlock : 256) k_sampl
             cplx<R> p;
             int pe;
             U.ratio12(d, l, f0, s0, f1, s1, p, pe);
-            // log2 |psi'/psi|^2: group sum of the lanes' log2 |p|^2, plus the
-            // visible-bias term 2 Re(-2 sum sigma_f c_f) / ln 2
-            R lp = M<R>::log2(norm2(p)) + (R)(2 * pe);
-            R lr2 = group_sum<L>(lp);
             R bre = (-2 * s0) * l.rb[f0].re;
             if (f1 >= 0) bre += (-2 * s1) * l.rb[f1].re;
-            lr2 += (R)2.8853900817779268 * bre;  // 2 / ln 2
-            if constexpr (PF) {
-                cplx<R> q = pf_ratio2<R, true>(l.pf, pv, st, __builtin_amdgcn_readfirstlane(f0),
-                                               __builtin_amdgcn_readfirstlane(f1), ln, pp);
-                lr2 += M<R>::log2(norm2(q));
+            constexpr R kBias = (R)2.8853900817779268;  // 2 / ln 2: visible-bias term 2 Re(-2 sum sigma_f c_f)
+            bool take;
+            if constexpr (sizeof(R) == 8) {
+                // u < |psi'/psi|^2 as u / 2^bias < group product of the lanes'
+                // |p|^2, as mantissa and exponent (no lane's factor may make
+                // the product leave the range)
+                const R b2 = kBias * bre, bt = b2 > 1e6 ? 1e6 : b2 < -1e6 ? -1e6 : b2, bi = __builtin_rint(bt);
+                const R lhs = uu * M<R>::exp2(bi - bt);
+                const R n2 = norm2(p);
+                R pm = frexp_m(n2);
+                pe = frexp_e(n2);
+                group_prod<L>(pm, pe);
+                pe += (int)bi;
+                if constexpr (PF) {
+                    const cplx<R> q = pf_ratio2<R, true>(l.pf, pv, st, __builtin_amdgcn_readfirstlane(f0),
+                                                         __builtin_amdgcn_readfirstlane(f1), ln, pp);
+                    const R q2 = norm2(q);
+                    pm *= frexp_m(q2);
+                    pe += frexp_e(q2);
+                }
+                take = lhs < M<R>::ldexp(pm, pe);
+            } else {
+                // log2 |psi'/psi|^2: group sum of the lanes' log2 |p|^2, plus the bias
+                R lp = M<R>::log2(norm2(p)) + (R)(2 * pe);
+                R lr2 = group_sum<L>(lp);
+                lr2 += kBias * bre;
+                if constexpr (PF) {
+                    cplx<R> q = pf_ratio2<R, true>(l.pf, pv, st, __builtin_amdgcn_readfirstlane(f0),
+                                                   __builtin_amdgcn_readfirstlane(f1), ln, pp);
+                    lr2 += M<R>::log2(norm2(q));
+                }
+                take = uu < M<R>::exp2(lr2);
             }
-            if (uu < M<R>::exp2(lr2)) {
+            if (take) {
                 U.accept12(d, l, f0, s0, f1, s1);
                 if constexpr (PF) pf_accept(l.pf, pv, pp, ln);
                 st[f0 >> 6] ^= (uint64_t)1 << (f0 & 63);
