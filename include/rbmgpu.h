@@ -69,11 +69,13 @@ typedef struct rbmgpu_config {
     int32_t lanes_per_chain; /* 0: autotune; 8/16/32/64: lane-group sampler with that
                                 many lanes per chain; -1: one chain per wavefront
                                 (FP32 only) */
-    int32_t keep_o;          /* 1: always materialise the O matrix.  0:
-                                a basic RBM in FP32 uses the structured
-                                S.x (O never formed, rbmgpu_get_samples
-                                cannot return O); other machines
-                                materialise O regardless */
+    int32_t keep_o;          /* 1: the O matrix can be read.  0: a basic RBM
+                                in FP32 uses the structured S.x (O never
+                                formed, rbmgpu_get_samples cannot return
+                                O).  Other machines always have O: the
+                                symmetric one with the samples, a basic RBM
+                                (FP64, Pfaffian factor, keep_o = 1) when it
+                                is first read */
     /* ---- learned proposal (no counterpart in the reference): cluster
      * flips drawn by a network z(s) = W2 relu(W1 s + b1) + b2 under
      * Metropolis-Hastings; FP32 machines without the Pfaffian factor */

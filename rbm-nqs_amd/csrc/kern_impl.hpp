@@ -765,7 +765,8 @@ __global__ void __launch_bounds__(PF && sizeof(R) == 4 ? kPfBlock : 256) k_sampl
                 if constexpr (PF) {
                     cplx<R> q = pf_ratio2<R, true>(l.pf, pv, st, __builtin_amdgcn_readfirstlane(f0),
                                                    __builtin_amdgcn_readfirstlane(f1), ln, pp);
-                    lr2 += M<R>::log2(norm2(q));
+                    // norm2 with its rounding written out: one ulp here turns a decision in 2e8
+                    lr2 += M<R>::log2(__builtin_fmaf(q.im, q.im, q.re * q.re));
                 }
                 take = uu < M<R>::exp2(lr2);
             }
