@@ -7,6 +7,6 @@ bool sx_ofree_ok(int real_size, int N, int M, int64_t ld, int npf) {
     // (16-wave blocks have no instance for N >= 32, kOfWide none for the Pfaffian block)
     const int mode = of_mode(N, M);
     if ((w != 4 && mode != kOfN32) || (mode == kOfWide && npf > 0)) return false;
-    return real_size == 4 ? of_ok<float>(N, M, (int)ld, npf, w) : of_ok<double>(N, M, (int)ld, npf, w);
+    return of_ok(real_size, N, M, (int)ld, npf, w);
 }
 }

@@ -22,6 +22,7 @@
 
 #include "dev_common.hpp"
 #include "kern_api.hpp"
+#include "ofree_index.hpp"
 
 namespace rbmgpu {
 
@@ -1273,39 +1274,12 @@ __global__ void __launch_bounds__(64 * WAVES) k_sx_partial(SxArgs<R> a) {
 //    (508 us with LDS reads at the size above);
 //  * otherwise, and for the biases, from the row staged in LDS.
 // The sign is +-1 with the sign bit shifted out of the (wave-uniform) state.
-// rows per step: 4, or 2 where the accumulators leave no registers for more
-// (blocks of 16 waves: 128 per lane; FP64 rows of over 1024 entries)
-template <typename R>
-__host__ __device__ constexpr int of_rows(int waves, int ld) {
-    return waves == 16 || (sizeof(R) == 8 && ld > 1024) ? 2 : 4;
-}
-constexpr int kOfMaxN = 62;  // bit 62 of a masked state word is 0
-// MODE: spins in both halves of the state word, in the low half, B32
-constexpr int kOfWide = 0, kOfN32 = 1, kOfB32 = 2;
-__host__ __device__ inline int of_mode(int N, int M) {
-    return N > 32 ? kOfWide : N == 32 && M % 32 == 0 ? kOfB32 : kOfN32;
-}
-__host__ __device__ inline int of_pad(int ld) { return (ld + 127) / 128 * 128; }
-__host__ __device__ inline int of_xs(int ld, int npf) { return of_pad(ld) + (npf + 1) / 2 * 2; }
-// LDS: x and the waves' rows, then two rows of sums
-template <typename R>
-__host__ __device__ inline size_t of_lds(int ld, int M, int npf, int waves) {
-    const size_t loop = (size_t)of_xs(ld, npf) + (size_t)waves * of_rows<R>(waves, ld) * (M + 1);
-    return (loop > 2 * (size_t)ld ? loop : 2 * (size_t)ld) * sizeof(cplx<R>);
-}
-// basic RBMs whose pairs never straddle two units (even N and M), the biases
-// within the first pair, at least two of the 4-wave blocks' LDS per CU
-template <typename R>
-__host__ __device__ inline bool of_ok(int N, int M, int ld, int npf, int waves) {
-    return N <= kOfMaxN && N % 2 == 0 && M % 2 == 0 && N + M <= 128 &&
-           of_lds<R>(ld, M, npf, waves) <= (waves == 16 ? 163840 : 81920);
-}
-
+// (rows per step, LDS and the places of a lane's entries: ofree_index.hpp)
 template <typename R, int ZM, int WAVES, int MODE, bool PF>
 __global__ void __launch_bounds__(64 * WAVES, WAVES == 16 ? 4 : 2) k_sx_ofree(SxArgs<R> a) {
     extern __shared__ __align__(16) char smem[];
     if (a.status && a.status->done) return;
-    constexpr int RW = of_rows<R>(WAVES, 128 * ZM);
+    constexpr int RW = of_rows(sizeof(R), WAVES, 128 * ZM);
     constexpr bool B32 = MODE == kOfB32;
     const int N = a.N, M = a.M, NM = N + M, rs = M + 1;
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1328,12 +1302,9 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES == 16 ? 4 : 2) k_sx_ofree(Sx
     // block), and a sum that starts at +0 keeps its bits.  Pair 0 holds the
     // biases (N + M <= 128): its places in the row, the spin of its signs (62:
     // +1); the unit and spin of pair 1 advance by 128 entries from pair to pair
-    const int q0 = 2 * lane - NM;
-    const int e0 = q0 >= 0 ? q0 / N : 2 * lane < N ? M : 2 * lane - N;
-    const int e1 = q0 >= 0 ? e0 : 2 * lane < N ? M : 2 * lane - N + 1;
-    const int ej = q0 >= 0 ? q0 - e0 * N : 2 * lane < N ? 2 * lane : 62;
-    const int j1 = (q0 + 128) % N, du = 128 / N, dj = 128 % N;
-    int uj = (q0 + 128) / N | j1 << 16;
+    const OfLane at = of_lane(lane, N, M);
+    const int e0 = at.e0, e1 = at.e1, ej = at.ej, j1 = at.j1, du = 128 / N, dj = 128 % N;
+    int uj = at.u1 | j1 << 16;
     cplx<R> z[2 * ZM];
 #pragma unroll
     for (int i = 0; i < 2 * ZM; i++) z[i] = {0, 0};
@@ -1417,12 +1388,7 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES == 16 ? 4 : 2) k_sx_ofree(Sx
                 j = uj >> 16;
                 return;
             }
-            u = min(u + du, M);  // past the end: x = 0 there
-            j += dj;
-            if (j >= N) {
-                j -= N;
-                u = min(u + 1, M);
-            }
+            of_next(u, j, du, dj, N, M);
         };
         // ---- y_r = O_r . x
         cplx<R> dot[RW];

@@ -101,8 +101,8 @@ hipError_t launch_o_partial(const MomArgs<R>& a, int blocks, hipStream_t st) {
 template <typename R, int ZM, int WAVES, int MODE, bool PF>
 static hipError_t sx_ofree_go(const SxArgs<R>& a, int blocks, hipStream_t st) {
     const int npf = a.P - a.P_rbm;
-    const size_t lds = of_lds<R>(a.ld, a.M, npf, WAVES);
-    if (!of_ok<R>(a.N, a.M, a.ld, npf, WAVES)) return hipErrorInvalidValue;
+    const size_t lds = of_lds(sizeof(R), a.ld, a.M, npf, WAVES);
+    if (!of_ok(sizeof(R), a.N, a.M, a.ld, npf, WAVES)) return hipErrorInvalidValue;
     if (lds > 65536) {
         hipError_t e = hipFuncSetAttribute((const void*)k_sx_ofree<R, ZM, WAVES, MODE, PF>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);

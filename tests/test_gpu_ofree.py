@@ -48,3 +48,16 @@ def test_ofree_moments_and_product(model, n, alpha, extra, prec, S):
     assert np.max(np.abs(g.get_samples(O=True)[2] - O)) <= tol * np.abs(O).max()
     g.load_samples(st[: S // 2])  # a smaller set: O follows it
     assert np.max(np.abs(g.get_samples(O=True)[2] - O[:, : S // 2])) <= tol * np.abs(O).max()
+
+
+# machines whose last pair of entries reaches past the last unit (N = 8 with 8,
+# 16 and 24 units, 2 x 3 cells with 12), through more than one step of a block's waves
+SMALL = [("toric", 2, 1, ""), ("kitaev", 2, 2, ""), ("toric", 2, 2, ""), ("kitaev", 2, 3, ""),
+         ("kitaev", 2, 1, "[model]\nn_cells_b = 3\n")]
+
+
+@pytest.mark.parametrize("model,n,alpha,extra", SMALL)
+@pytest.mark.parametrize("prec", [64, 32])
+@pytest.mark.parametrize("S", [3, 37, 1501])
+def test_ofree_past_the_last_unit(model, n, alpha, extra, prec, S):
+    test_ofree_moments_and_product(model, n, alpha, extra, prec, S)
