@@ -177,6 +177,7 @@ namespace {
         hipError_t e_ = (x);                                                       \
         if (e_ != hipSuccess) {                                                    \
             ctx->err = std::string(#x) + ": " + hipGetErrorString(e_);             \
+            (void)hipGetLastError(); /* or the next launch's check reports it */   \
             return -2;                                                             \
         }                                                                          \
     } while (0)
@@ -299,6 +300,10 @@ Terms terms(const rbmgpu_ctx* c) {
 int ensure_samples(rbmgpu_ctx* c, int64_t S) {
     rbmgpu_ctx* ctx = c;
     if (S <= c->cap) return 0;
+    // an allocation below may fail: no capacity and no sample set are left then
+    c->cap = 0;
+    c->S = 0;
+    c->have_chains = c->weighted = c->learned_epoch = c->moments_valid = false;
     if (int rc = dalloc(ctx, &c->d_states, S * c->nw * sizeof(uint64_t))) return rc;
     if (int rc = dalloc(ctx, &c->d_obs, S * 2 * c->n_groups * sizeof(double))) return rc;
     if (int rc = dalloc(ctx, &c->d_T, S * c->H * 2 * rsize(c))) return rc;
@@ -513,6 +518,7 @@ int learn_pack(rbmgpu_ctx* c) {
 int ensure_train(rbmgpu_ctx* c, int64_t B) {
     rbmgpu_ctx* ctx = c;
     if (B <= c->tr_cap) return 0;
+    c->tr_cap = 0;
     // S (B x N), A (B x Hn), dZ (B x N), dU (B x Hn), loss (B), w (B)
     if (int rc = dalloc(ctx, &c->d_tr, (size_t)B * (2 * c->N + 2 * c->Hn + 1) * sizeof(float))) return rc;
     if (int rc = dalloc(ctx, &c->d_tst, (size_t)B * c->nw * sizeof(uint64_t))) return rc;
@@ -628,6 +634,7 @@ int ensure_O(rbmgpu_ctx* c) {
     rbmgpu_ctx* ctx = c;
     if (!c->ofree || c->o_built || c->S == 0) return 0;
     if (c->S > c->o_cap) {
+        c->o_cap = 0;
         if (int rc = dalloc(ctx, &c->d_O, c->S * c->ld * 2 * rsize(c))) return rc;
         c->o_cap = c->S;
     }
@@ -1313,6 +1320,7 @@ int struct_moments(rbmgpu_ctx* c) {
                              (vch + kVarWaves - 1) / kVarWaves));
     const int64_t vneed = nvb * L * (int64_t)sizeof(double);
     if (vneed > c->varpart_cap) {
+        c->varpart_cap = 0;
         if (int rc = dalloc(ctx, &c->d_varpart, vneed)) return rc;
         c->varpart_cap = vneed;
     }
@@ -1374,6 +1382,7 @@ int ensure_sx(rbmgpu_ctx* c) {
     if (int rc = sx_layout(c, &blocks, &need)) return rc;
     c->sx_blocks = blocks;
     if (need > c->sxpart_cap) {
+        c->sxpart_cap = 0;
         if (int rc = dalloc(ctx, &c->d_sxpart, need)) return rc;
         c->sxpart_cap = need;
     }
@@ -1528,6 +1537,7 @@ int compute_moments(rbmgpu_ctx* c) {
     const int64_t nblk = nb > 1 ? nb * per_bin : (c->S + chunk - 1) / chunk;
     const int64_t pneed = nblk * (3 + 2 * c->n_groups) * (int64_t)sizeof(double);
     if (pneed > c->epart_cap) {
+        c->epart_cap = 0;
         if (int rc = dalloc(ctx, &c->d_epart, pneed)) return rc;
         c->epart_cap = pneed;
     }
@@ -1551,6 +1561,7 @@ int compute_moments(rbmgpu_ctx* c) {
         }
         int64_t need = blocks * c->P * kOPartRow;
         if (need > c->part_cap) {
+            c->part_cap = 0;
             if (int rc = dalloc(ctx, &c->d_part, need * sizeof(double))) return rc;
             c->part_cap = need;
         }
@@ -1570,6 +1581,7 @@ int compute_moments(rbmgpu_ctx* c) {
 int ensure_eval(rbmgpu_ctx* c, int64_t n) {
     rbmgpu_ctx* ctx = c;
     if (n <= c->ev_cap) return 0;
+    c->ev_cap = 0;
     if (int rc = dalloc(ctx, &c->d_evst, n * c->nw * sizeof(uint64_t))) return rc;
     if (int rc = dalloc(ctx, &c->d_evout, n * 2 * sizeof(double))) return rc;
     c->ev_cap = n;
@@ -1826,6 +1838,7 @@ int build_S_t(rbmgpu_ctx* c, double r1, double r2, double rd, int mode, const do
     const int64_t gbytes = (int64_t)a.npairs * 64 * 64 * (int64_t)sizeof(double);
     const int64_t need = gbytes + (int64_t)a.ksplit * a.npairs * 64 * 64 * (int64_t)sizeof(R);
     if (need > c->gpart_cap) {
+        c->gpart_cap = 0;
         if (int rc = dalloc(ctx, &c->d_gpart, need)) return rc;
         c->gpart_cap = need;
     }
@@ -2612,6 +2625,9 @@ int rbmgpu_full_epoch(rbmgpu_ctx* c, int32_t parallel_bits) {
     if (int rc = ensure_samples(c, S)) return rc;
     const int nb = (int)std::min<int64_t>((S + 255) / 256, 1024);
     if (S > c->w_cap) {
+        c->w_cap = 0;
+        c->S = 0;
+        c->weighted = c->moments_valid = false;
         if (int rc = dalloc(ctx, &c->d_w, S * sizeof(double))) return rc;
         if (int rc = dalloc(ctx, &c->d_wsx, S * sizeof(double))) return rc;
         if (int rc = dalloc(ctx, &c->d_lp, S * 2 * sizeof(double))) return rc;
