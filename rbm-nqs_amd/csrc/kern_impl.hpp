@@ -111,15 +111,15 @@ template <typename R, int L, int K>
 struct Units {
     int a[K], s[K];  // alpha and symmetry index per unit, a < 0: padding
     cplx<R> th[K], tn[K];
-    // K <= 4 in FP32, K <= 2 in FP64 (more units would cost occupancy): cosh and
+    // FP32 (K <= 4; more units would cost occupancy): cosh and
     // sinh of the last ratio12 flip set's delta per unit and the unit's
     // ratio factor cosh(theta + delta) / cosh(theta), kept for accept12's
     // tanh update
-    static constexpr bool kMob = sizeof(R) == 4 ? K <= 4 : K <= 2;
-    // more units per lane: the same Mobius step, its cosh / sinh
+    static constexpr bool kMob = sizeof(R) == 4 && K <= 4;
+    // FP32 with more units per lane: the same Mobius step, its cosh / sinh
     // factors reloaded from the tables at the (less frequent) accepted move
     // instead of kept in registers from the ratio
-    static constexpr bool kMobR = !kMob;
+    static constexpr bool kMobR = sizeof(R) == 4 && !kMob;
     cplx<R> kc[kMob ? K : 1], ks[kMob ? K : 1], kr[kMob ? K : 1];
     // K <= 2, L <= 32 (the Pfaffian shapes have L = 64 and no registers to
     // spare): W entries of the last ratio12 flip set, loaded with its C
@@ -242,12 +242,14 @@ struct Units {
             if (sizeof(R) == 4 && (u & 3) == 3) renorm(p, pe);
         }
     }
-    // after a sweep: tanh from theta again (the accepted moves update tanh
-    // incrementally, see accept12_w)
+    // FP32 (kMob) after a sweep: tanh from theta again (the accepted moves
+    // update tanh incrementally, see accept12_w)
     __device__ void resync() {
+        if constexpr (kMob || kMobR) {
 #pragma unroll
-        for (int u = 0; u < K; u++)
-            if (a[u] >= 0) tn[u] = ctanh(th[u]);
+            for (int u = 0; u < K; u++)
+                if (a[u] >= 0) tn[u] = ctanh(th[u]);
+        }
     }
     // generic flip set: sites fl[i] for i < 8 with bit i of mask set
     __device__ void ratio_mask(const Dims& d, const Lds<R>& l, const int* fl, const R* sg, int mask,
@@ -294,14 +296,16 @@ struct Units {
         else
             accept12_w(d, l, l.Wg, f0, s0, f1, s1);
     }
-    // tanh is updated from the ratio12 of the same flip set:
+    // FP64 recomputes tanh(theta): the chains follow the oracle's state for
+    // state.  (The update below, whose error over a sweep grows with the
+    // weights -- 1e-15 at 0.05, 3e-13 at 0.3, all digits from about 1.5 on --
+    // moved chains there, and is left to FP32.)  FP32 updates tanh from the
+    // ratio12 of the same flip set:
     // tanh(theta + delta) = (t cosh delta + sinh delta) / (cosh delta +
     // t sinh delta), whose denominator is the unit's ratio factor (a move
     // is accepted with probability |prod of factors|^2, so a vanishing
     // factor is almost never divided by); resync() restores tanh(theta)
-    // after every sweep, so rounding builds up over one sweep at most, and
-    // what is written of a kept sample is tanh(theta) itself.  theta moves by
-    // the same sums as ever
+    // after every sweep, so rounding builds up over one sweep at most
     __device__ void accept12_w(const Dims& d, const Lds<R>& l, const cplx<R>* W, int f0, R s0, int f1, R s1) {
         if constexpr (!kPreW) {  // unit by unit
 #pragma unroll
@@ -329,7 +333,7 @@ struct Units {
                 if constexpr (kMobR) {
                     // tanh(theta + delta) = (t cosh delta + sinh delta) / (cosh delta + t sinh delta)
                     const cplx<R> num = tn[u] * ch + sh, r = ch + tn[u] * sh;
-                    const R inv = rcp(r.re * r.re + r.im * r.im);
+                    const R inv = __builtin_amdgcn_rcpf(r.re * r.re + r.im * r.im);
                     tn[u] = {(num.re * r.re + num.im * r.im) * inv, (num.im * r.re - num.re * r.im) * inv};
                 } else {
                     update_tanh(u);
@@ -346,12 +350,14 @@ struct Units {
         }
     }
     __device__ void update_tanh(int u) {
-        const cplx<R> num = tn[u] * kc[u] + ks[u], r = kr[u];
-        const R inv = rcp(r.re * r.re + r.im * r.im);
-        tn[u] = {(num.re * r.re + num.im * r.im) * inv, (num.im * r.re - num.re * r.im) * inv};
+        if constexpr (kMob) {
+            const cplx<R> num = tn[u] * kc[u] + ks[u], r = kr[u];
+            const R inv = __builtin_amdgcn_rcpf(r.re * r.re + r.im * r.im);
+            tn[u] = {(num.re * r.re + num.im * r.im) * inv, (num.im * r.re - num.re * r.im) * inv};
+        } else {
+            tn[u] = ctanh(th[u]);
+        }
     }
-    static __device__ float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
-    static __device__ double rcp(double x) { return 1 / x; }
 };
 
 // psi(sigma')/psi(sigma) for the sites of a term selected by mask: the
@@ -650,9 +656,9 @@ __device__ inline void eval_obs(const Dims& d, const Lds<R>& l, const Units<R, L
 // slots), else one uniform site; accept if u < |psi'/psi|^2.  At kept
 // steps the local observables and tanh(theta) of the sample are written.
 // A chain is one dependent sequence of proposals, so with few chains the sampler
-// is bound by a proposal's latency: in FP64 the decision takes no logarithm and
-// the accepted move no exponential or sine (toric 4x4 symmetric, 64 chains, 450
-// sweeps: 13.9 -> 9.6 ms; basic, 4096 chains x 164 sweeps: 15.5 -> 12.3 ms).
+// is bound by a proposal's latency: in FP64 the decision takes no logarithm
+// (toric 4x4 symmetric, 64 chains, 450 sweeps: epoch 17.9 -> 16.0 ms; basic,
+// 4096 chains x 164 sweeps: 57.8 -> 57.1 ms).
 // With the Pfaffian factor in FP32 up to 8 chains share a block's tables: its
 // LDS lets one block per CU run (Kitaev 4x4), as two wavefronts per SIMD of 256
 // registers; in FP64 one of 512 registers.
@@ -741,8 +747,8 @@ __global__ void __launch_bounds__(PF && sizeof(R) == 4 ? kPfBlock : 256) k_sampl
             bool take;
             if constexpr (sizeof(R) == 8) {
                 // u < |psi'/psi|^2 as u / 2^bias < group product of the lanes'
-                // |p|^2, as mantissa and exponent (no lane's factor may make
-                // the product leave the range)
+                // |p|^2, as mantissa and exponent, so that the product stays in
+                // range whatever the lanes' factors are
                 const R b2 = kBias * bre, bt = b2 > 1e6 ? 1e6 : b2 < -1e6 ? -1e6 : b2, bi = __builtin_rint(bt);
                 const R lhs = uu * M<R>::exp2(bi - bt);
                 const R n2 = norm2(p);

@@ -38,3 +38,20 @@ def test_accept_fp64(model, n, rbm, alpha, lanes, big):
     st_o, e_o, _, _ = o.sample(seed=421390484, epoch=3, n_samples=m.n_samples, n_chains=m.n_chains)
     assert np.array_equal(st, st_o)
     assert np.max(np.abs(obs[:, 0] - e_o)) <= 1e-10 * (np.abs(e_o).max() + 1)
+
+
+# weights at which an incremental tanh loses its digits within a sweep
+@pytest.mark.parametrize("model,n,rbm,alpha,std", [("toric", 4, "basic", 2, 1.5), ("toric", 4, "symmetry", 1, 2.0),
+                                                   ("kitaev", 6, "symmetry", 2, 1.5), ("kitaev", 6, "symmetry", 2, 2.0)])
+def test_large_weights_fp64(model, n, rbm, alpha, std):
+    print(f"[gpu-test] large weights {model}{n} {rbm} std={std}", flush=True)
+    spec = ini(model, n, rbm=rbm, alpha=alpha, extra="[sampler]\nn_samples = 960\nmetropolis.n_chains = 48\n"
+               "metropolis.n_warmup_steps = 20\nmetropolis.bond_flips = 0.4\n")
+    m, o = rbmgpu.Model(spec), po.Oracle(spec)
+    p = random_params(np.random.default_rng(1), m.P, std)
+    o.set_params(p)
+    g = m.gpu(precision=64)
+    g.set_params(p)
+    g.sample_epoch(epoch=3)
+    st_o, _, _, _ = o.sample(seed=421390484, epoch=3, n_samples=m.n_samples, n_chains=m.n_chains)
+    assert np.array_equal(g.get_samples()[0], st_o)
