@@ -1978,11 +1978,20 @@ __global__ void __launch_bounds__(256) k_wsx(const double* w, int64_t S, const d
         wsx[k] = (double)S * w[k] / W;
 }
 
+// the host's side of a sampled epoch: what the device's buffers hold once it
+// has run, eagerly or as a replayed graph (whose host code does not run again)
+void epoch_state(rbmgpu_ctx* c) {
+    c->S = c->n_samples;
+    c->have_chains = true;
+    c->weighted = false;
+    c->learned_epoch = c->Hn && c->lam > 0;
+    c->moments_valid = false;
+}
+
 // one sampling epoch on the stream: all chains, the kept samples' local
 // observables and (materialised path) the O matrix; buffers allocated
 int sample_body(rbmgpu_ctx* c, uint32_t epoch) {
     rbmgpu_ctx* ctx = c;
-    c->weighted = false;
     if (int rc = zero_async(c, c->d_obs, c->n_samples * 2 * c->n_groups * sizeof(double))) return rc;
     if (int rc = record(c, 0)) return rc;
     int rc = 0;
@@ -1997,14 +2006,10 @@ int sample_body(rbmgpu_ctx* c, uint32_t epoch) {
     }
     if (rc) return rc;
     if (int rc2 = record(c, 1)) return rc2;
-    c->learned_epoch = c->Hn && c->lam > 0;
-    c->S = c->n_samples;
-    c->have_chains = true;
+    epoch_state(c);
     rc = c->prec == RBMGPU_FP32 ? run_build_O<float>(c) : run_build_O<double>(c);
     if (rc) return rc;
-    if (int rc2 = record(c, 2)) return rc2;
-    c->moments_valid = false;
-    return 0;
+    return record(c, 2);
 }
 
 
@@ -2540,7 +2545,9 @@ int rbmgpu_train_epoch(rbmgpu_ctx* c, uint32_t epoch, const rbmgpu_sr_params* sp
             if (g.first == budget) ex = g.second;
         if (ex) {
             HIPCK(hipGraphLaunch(ex, c->stream));
-            c->o_built = c->train_dense == 1;  // the replay's samples; O only if S was built from it
+            epoch_state(c);
+            c->o_built = c->train_dense == 1;  // O only if S was built from it
+            if (int rc = ensure_sx(c)) return rc;  // this set's layout, for train_more
         } else {
             // this epoch runs eagerly (allocating what it needs), then the
             // same body is captured for the following epochs
