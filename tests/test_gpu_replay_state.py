@@ -35,14 +35,19 @@ def test_replay_after_another_set(rbm, prec, explicit, between):
     for graph in (True, False):
         g = m.gpu(precision=prec, lanes=64)
         g.set_params(p)
+
+        def other():
+            if between == "load":
+                g.load_samples(few)
+            else:
+                g.full_epoch()
+            g.apply_S(p, 0.1, 1e-4, 0.0)
+
+        other()  # every buffer is there before the graph: it is not captured again
         for e in (1, 2):
             r = g.train_epoch(e, 1e-2, 0.1, 1e-4, 0.0, max_iter=100, rtol=1e6, graph=graph)
             assert r["itn"] < 6
-        if between == "load":
-            g.load_samples(few)
-            g.apply_S(p, 0.1, 1e-4, 0.0)
-        else:
-            g.full_epoch()
+        other()
         r = g.train_epoch(3, 1e-2, 0.1, 1e-4, 0.0, max_iter=100, graph=graph)
         assert r["itn"] > 8 and r["graph"] == graph
         assert g.n_samples() == 4096
