@@ -113,7 +113,12 @@ struct EvalArgs {
     int n_flips;
 };
 
-// log psi of given states without the Pfaffian factor (kern_logpsi.hip)
+// log psi of given states without the Pfaffian factor (kern_logpsi.hip): a
+// block of kLpWaves wavefronts with kLpStatic bytes of sums and up to kLpTables
+// bytes of tables in its 64 KiB of LDS; the symmetry permutations have to fit
+constexpr int kLpWaves = 4;
+constexpr size_t kLpStatic = kLpWaves * 16 * 2 * sizeof(double), kLpTables = 65536 - kLpStatic;
+inline bool logpsi_tables_fit(int ns, int N) { return ns == 1 || (size_t)ns * N <= kLpTables; }
 template <typename R>
 struct LogpsiArgs {
     int64_t n;

@@ -55,12 +55,11 @@ __device__ inline void sc(float y, float& s, float& c) { ::sincosf(y, &s, &c); }
 // the argument of (re, im) lies in (0, pi]
 __device__ inline bool upper(double re, double im) { return im > 0 || (im == 0 && re < 0 && !signbit(im)); }
 
-constexpr int kLpWaves = 4;
-
 template <typename R>
 __global__ void __launch_bounds__(64 * kLpWaves) k_logpsi(LogpsiArgs<R> a) {
     extern __shared__ __align__(16) char smem[];
     __shared__ double red[kLpWaves][16][2];
+    static_assert(sizeof(red) == kLpStatic, "counted in the LDS budget");
     const int N = a.N, H = a.H, na = a.na, ns = a.ns;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, n = lane & 15, g = lane >> 4;
     cplx<R>* Wl = reinterpret_cast<cplx<R>*>(smem);
@@ -156,10 +155,10 @@ template <typename R>
 hipError_t launch_logpsi(LogpsiArgs<R> a, int n_cu, hipStream_t st) {
     if (a.n < 1 || a.N < 1 || a.H < 1 || a.nw > 2) return hipErrorInvalidValue;
     const size_t wb = (size_t)a.N * a.na * sizeof(cplx<R>), pb = a.ns > 1 ? (size_t)a.ns * a.N : 0;
-    a.w_lds = wb + pb <= 65536;  // else from memory (caches)
+    if (!logpsi_tables_fit(a.ns, a.N)) return hipErrorInvalidValue;
+    a.w_lds = wb + pb <= kLpTables;  // else from memory (caches)
     const size_t lds = (a.w_lds ? wb : 0) + pb;
-    if (lds > 65536) return hipErrorInvalidValue;
-    const int64_t per_cu = std::max<int64_t>(1, std::min<int64_t>(8, 163840 / (int64_t)(lds + 1024)));
+    const int64_t per_cu = std::max<int64_t>(1, std::min<int64_t>(8, 163840 / (int64_t)(lds + kLpStatic)));
     const int64_t blocks = std::min<int64_t>((a.n + 15) / 16, per_cu * n_cu);
     hipLaunchKernelGGL(k_logpsi<R>, dim3((unsigned)blocks), dim3(64 * kLpWaves), lds, st, a);
     return hipGetLastError();

@@ -1588,9 +1588,6 @@ int ensure_eval(rbmgpu_ctx* c, int64_t n) {
     return 0;
 }
 
-// k_logpsi keeps the symmetry permutations in LDS (at most 64 KiB)
-bool logpsi_tables_fit(const rbmgpu_ctx* c) { return c->nsymm == 1 || (int64_t)c->nsymm * c->N <= 65536; }
-
 template <typename R>
 int run_logpsi(rbmgpu_ctx* c, const uint64_t* d_states, int64_t n, double* logpsi) {
     rbmgpu_ctx* ctx = c;
@@ -1644,14 +1641,14 @@ int run_eval(rbmgpu_ctx* c, const uint64_t* d_states, int64_t n, double* logpsi,
     // other outputs -- sample sets, exact enumeration, whose weights |psi|^2
     // the SR solve amplifies -- a group of lanes per state, whose sums keep
     // their order.)
-    if (logpsi && !obs && !Tout && !ratio && !c->pf_rows && logpsi_tables_fit(c))
+    if (logpsi && !obs && !Tout && !ratio && !c->pf_rows && logpsi_tables_fit(c->nsymm, c->N))
         return run_logpsi<R>(c, d_states, n, logpsi);
     if constexpr (sizeof(R) == 4) {
         // sample sets in FP32: the tanh rows and observables through the wave
         // sampler's tables (basic RBM: k_eloc's observables), log psi by
         // k_logpsi.  FP64 sample sets keep the lane-group evaluation: its sums'
         // order reaches the SR solve, which amplifies a change of rounding.
-        if (Tout == c->d_T && obs == c->d_obs && !ratio && wave_ok(c) && (!logpsi || logpsi_tables_fit(c))) {
+        if (Tout == c->d_T && obs == c->d_obs && !ratio && wave_ok(c) && (!logpsi || logpsi_tables_fit(c->nsymm, c->N))) {
             SampArgs<float> w = samp_args<float>(c, 0, 512, n, 0);
             const int K = (c->H + 63) / 64;
             w.npair = c->nsymm > 1 ? c->npair : 0;

@@ -36,3 +36,10 @@ def test_logpsi_tiles(model, n, rbm, alpha, prec, std):
         got = g.eval_logpsi(st[:S])
         err = np.abs(got - want[:S])
         assert np.all(err <= tol * (1 + np.abs(want[:S]))), (S, err.max())
+
+
+# 32 x 128 complex weights in FP64, 32 x 256 in FP32: 64 KiB, which with the
+# kernel's own sums do not fit the 64 KiB of a launch without opting in
+@pytest.mark.parametrize("alpha,prec", [(4, 64), (8, 32)])
+def test_logpsi_tables_of_64_kib(alpha, prec):
+    test_logpsi_tiles("toric", 4, "basic", alpha, prec, 0.05)
