@@ -74,8 +74,12 @@ typedef struct rbmgpu_config {
                                 formed, rbmgpu_get_samples cannot return
                                 O).  Other machines always have O: the
                                 symmetric one with the samples, a basic RBM
-                                (FP64, Pfaffian factor, keep_o = 1) when it
-                                is first read */
+                                (FP64, Pfaffian factor, keep_o = 1) from
+                                the call that first reads it on (get_samples
+                                with O, build_S, cg-single, direct): that
+                                call allocates and fills samples x params
+                                complex, and is the one that fails when
+                                they do not fit */
     /* ---- learned proposal (no counterpart in the reference): cluster
      * flips drawn by a network z(s) = W2 relu(W1 s + b1) + b2 under
      * Metropolis-Hastings; FP32 machines without the Pfaffian factor */

@@ -635,7 +635,11 @@ int ensure_O(rbmgpu_ctx* c) {
     if (!c->ofree || c->o_built || c->S == 0) return 0;
     if (c->S > c->o_cap) {
         c->o_cap = 0;
+        // captured epochs hold O's address only where they build S from it:
+        // the others stay
+        const uint64_t gen = c->gen;
         if (int rc = dalloc(ctx, &c->d_O, c->S * c->ld * 2 * rsize(c))) return rc;
+        if (c->train_dense != 1) c->gen = gen;
         c->o_cap = c->S;
     }
     if (int rc = c->prec == RBMGPU_FP32 ? enqueue_build_O<float>(c) : enqueue_build_O<double>(c)) return rc;

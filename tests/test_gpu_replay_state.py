@@ -57,3 +57,26 @@ def test_replay_after_another_set(rbm, prec, explicit, between):
         out.append((g.get_params(), r["mean"], r["n_bins"], st, obs, acc, q["mean"], q["o_mean"], y))
     for a, b in zip(*out):
         assert np.array_equal(a, b)
+
+
+def test_reading_O_keeps_the_graph():
+    """O of a basic FP64 machine is built when it is read.  Its buffer is not in
+    the captured epoch, so reading it must not cost the graph: a replay records
+    no timing events, and kernel_times shows those of the last eager epoch."""
+    print("[gpu-test] reading O between replays", flush=True)
+    m = rbmgpu.Model(ini("toric", 3, alpha=2, extra="[sampler]\nn_samples = 2000\nmetropolis.n_chains = 100\n"
+                         "metropolis.n_warmup_steps = 10\n[gpu]\nexplicit_s = false\n"))
+    g = m.gpu(precision=64, lanes=64)
+    g.set_params(random_params(np.random.default_rng(8), m.P, 0.05))
+
+    def epoch(e):
+        g.train_epoch(e, 1e-3, 0.1, 1e-4, 0.0, max_iter=8)
+        g.reduce()
+        return g.kernel_times()
+
+    epoch(1)
+    before = epoch(2)
+    O = g.get_samples(O=True)[2]
+    assert np.abs(O).max() > 0
+    after = epoch(3)
+    assert after["sample"] == before["sample"]
