@@ -44,7 +44,9 @@ struct WaveLds {
     const float2* fac;  // per entry: matrix element x exp(-2 sum_f sigma_f c_f) of its flipped sites
 };
 
-template <int K>
+// EXACT (given states): the entry factors' exponential and sine to FP32's last
+// bits, as the lane-group evaluation forms them
+template <int K, bool EXACT = false>
 __device__ inline WaveLds wave_stage(const SampArgs<float>& a, char* smem) {
     const Dims& d = a.d;
     const int ne = wave_n_entries(d), nreal = d.N * d.n_alpha, na = d.n_alpha;
@@ -113,11 +115,16 @@ __device__ inline WaveLds wave_stage(const SampArgs<float>& a, char* smem) {
                         br += m2 * c.re;
                         bi += m2 * c.im;
                     }
-                float sn, cs;
-                sincos_f(bi, sn, cs);
-                const float ex = __expf(br);
-                const cplx<float> f = cplx<float>{(float)T.val[2 * e], (float)T.val[2 * e + 1]} *
-                                      cplx<float>{ex * cs, ex * sn};
+                cplx<float> ex;
+                if constexpr (EXACT) {
+                    ex = cexp(cplx<float>{br, bi});
+                } else {
+                    float sn, cs;
+                    sincos_f(bi, sn, cs);
+                    const float m = __expf(br);
+                    ex = {m * cs, m * sn};
+                }
+                const cplx<float> f = cplx<float>{(float)T.val[2 * e], (float)T.val[2 * e + 1]} * ex;
                 fac[e] = make_float2(f.re, f.im);
             }
         }
@@ -388,7 +395,11 @@ struct WaveUnits {
 // the pair-table path, which then runs term after term with no dependent
 // table reads in between (the codes come by v_readlane); the other terms
 // take the generic path.
-template <int K, bool SYM>
+//
+// EXACT (given states): the lane's partial is scaled before the factor comes
+// in, so that a factor near FP32's limit (visible biases from about 20 on)
+// does not overflow with it.
+template <int K, bool SYM, bool EXACT = false>
 __device__ inline void wave_obs(const Dims& d, const WaveLds& l, const WaveUnits<K, SYM>& U, uint64_t st0,
                                 uint64_t st1, int npair, double* out) {
     constexpr int B = 4, J = 2;
@@ -416,6 +427,11 @@ __device__ inline void wave_obs(const Dims& d, const WaveLds& l, const WaveUnits
         nb = 0;
     };
     auto push = [&](cplx<float> p, int pe, int e) __attribute__((always_inline)) {
+        if constexpr (EXACT) {
+            renorm(p, pe);
+            p = {0.5f * p.re, 0.5f * p.im};  // |re| + |im| <= 1
+            pe++;
+        }
         if (U.ln == 0) p = p * cplx<float>{l.fac[e].x, l.fac[e].y};
         renorm(p, pe);
 #pragma unroll
@@ -696,7 +712,7 @@ template <int K, bool SYM>
 __global__ void __launch_bounds__(kWaveEvalBlock) k_eval_wave(SampArgs<float> a) {
     extern __shared__ __align__(16) char smem[];
     const Dims d = a.d;
-    const WaveLds l = wave_stage<K>(a, smem);
+    const WaveLds l = wave_stage<K, true>(a, smem);
     const int ln = threadIdx.x & 63;
     WaveUnits<K, SYM> U;
     U.init(d, l, ln, a.npair);
@@ -707,7 +723,7 @@ __global__ void __launch_bounds__(kWaveEvalBlock) k_eval_wave(SampArgs<float> a)
 #pragma unroll
         for (int u = 0; u < K; u++)
             if (u < K - 1 || U.vlast) a.Tout[k * d.H + ln + u * 64] = U.tn[u];
-        if (a.obs) wave_obs<K, SYM>(d, l, U, st0, st1, a.npair, a.obs + k * 2 * a.T.n_groups);
+        if (a.obs) wave_obs<K, SYM, true>(d, l, U, st0, st1, a.npair, a.obs + k * 2 * a.T.n_groups);
     }
 }
 

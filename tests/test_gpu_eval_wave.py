@@ -37,3 +37,25 @@ def test_eval_wave(model, n, rbm, alpha, extra, S):
     if rbm == "symmetry":
         O = o.derivative(st)
         assert np.max(np.abs(got[2] - O)) <= 1e-4 * np.abs(O).max()
+
+
+# visible biases whose factor exp(-4 c) of a bond flip comes near FP32's limit
+# (3.3e37 to 1.7e38): the energies, some 1e45, are within the doubles' range
+@pytest.mark.parametrize("n,alpha", [(2, 4), (3, 2), (4, 2), (6, 1), (6, 4)])
+@pytest.mark.parametrize("c", [21.8, -21.8, 22.0, -22.0, 22.15])
+def test_eval_wave_large_visible_bias(n, alpha, c):
+    print(f"[gpu-test] eval_wave kitaev {n} alpha={alpha} visible bias {c}", flush=True)
+    rng = np.random.default_rng(3)
+    spec = ini("kitaev", n, rbm="symmetry", alpha=alpha)
+    m, o = rbmgpu.Model(spec), po.Oracle(spec)
+    p = random_params(rng, m.P, 0.3)
+    p[: m.n_vb] = c + 0.3j
+    p = p.astype(np.complex64).astype(np.complex128)
+    o.set_params(p)
+    g = m.gpu(precision=32)
+    g.set_params(p)
+    st = po.random_states(np.random.default_rng(7), 64, m.N)
+    g.load_samples(st)
+    e, got = o.eloc(st), g.get_samples()[1][:, 0]
+    assert np.all(np.isfinite(got))
+    assert np.max(np.abs(got - e)) <= 1e-4 * np.abs(e).max()
