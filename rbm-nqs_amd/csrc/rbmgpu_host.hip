@@ -31,6 +31,7 @@ struct rbmgpu_ctx {
     int64_t P = 0, P_rbm = 0, ld = 0;  // ld: O row length (P rounded up to even)
     std::vector<int32_t> perm, basis, pb;
     int n_terms = 0, n_groups = 1, n_rowptr = 0, n_ent = 0, tk_max = 0, n_ratio = 0;
+    int n_pair_terms = 0;  // off-diagonal terms on a proposal bond (pair tables)
     int eloc_bpc = 0;  // resident k_eloc blocks per CU (0: not yet queried)
     // ---- sampler
     int n_chains = 1, warmup = 0, step = 1, prec = 64, lanes_req = 0, keep_o = 1;
@@ -1613,6 +1614,35 @@ int run_logpsi(rbmgpu_ctx* c, const uint64_t* d_states, int64_t n, double* logps
     return 0;
 }
 
+// whether n given FP32 states are faster through the wave sampler's tables
+// (k_eval_wave, for a basic RBM with k_eloc after it) than by groups of lanes.
+// Staging the tables and the second launch cost 5 to 25 us a call, so few
+// states have to be worth it (load_samples, us, lane groups / wave):
+//   symmetric, every off-diagonal term a pair-table entry: always (Kitaev 2x2
+//     1 state 44 / 42, 4x4 85 / 77, 6x6 alpha = 4 321 / 161; 65 536: 5964 / 2505)
+//   some terms (hexagons evaluated too): more than two units per lane always
+//     (6x6 alpha = 4: 481 / 390), else from 5120 (two state words: 8192) states on
+//     (4x4: 2048 states 145 / 145, 8192 0.75 of it; 6x6 alpha = 1: 4096 582 / 612)
+//   none (toric): one state word, at most two units per lane and 16384 states
+//     (4x4 alpha = 4: 4096 127 / 143, 16384 0.95; 5x5 alpha = 4 never: 2881 / 2996)
+//   basic, energies by k_eloc: from 5120 states on (toric 4x4 alpha = 2: 2048
+//     1.31, 5120 0.70 of it), with more than one unit per lane once n N reaches
+//     131072 (Kitaev 2x2 alpha = 16: 8192 1.21, 16384 0.94; 4x4 alpha = 3: 2048 1.16,
+//     4096 0.75)
+//   basic, energies inside: more than one unit per lane from 512 states on (6x6
+//     Kitaev: 64 185 / 214, 512 337 / 220), else n N from 262144 (3x3 with
+//     hexagons: 8192 1.05, 16384 0.94; 5x5: 8192 0.58)
+bool eval_wave_faster(const rbmgpu_ctx* c, int64_t n) {
+    if (c->nsymm > 1) {
+        const int pairs = c->npair > 0 ? c->n_pair_terms : 0;
+        if (pairs > 0 && pairs == c->n_ratio) return true;
+        if (pairs > 0) return c->H > 128 || n >= (c->nw == 1 ? 5120 : 8192);
+        return c->nw == 1 && c->H <= 128 && n >= 16384;
+    }
+    if (eloc_after(c)) return c->H > 64 ? n * c->N >= 131072 : n >= 5120;
+    return c->H > 64 ? n >= 512 : n * c->N >= 262144;
+}
+
 template <typename R>
 int run_eval(rbmgpu_ctx* c, const uint64_t* d_states, int64_t n, double* logpsi, double* obs, void* Tout,
              double* ratio, const int32_t* flips, int nf) {
@@ -1641,18 +1671,19 @@ int run_eval(rbmgpu_ctx* c, const uint64_t* d_states, int64_t n, double* logpsi,
                 if (shape_fits(c, kShapes[i]) && (!s.L || kShapes[i].L * kShapes[i].K < s.L * s.K)) s = kShapes[i];
     }
     if (!s.L) return fail(c, "no launch shape for this number of hidden units");
-    // log psi alone, for a caller that reads it: 16 states per tile.  (With
-    // other outputs -- sample sets, exact enumeration, whose weights |psi|^2
-    // the SR solve amplifies -- a group of lanes per state, whose sums keep
-    // their order.)
+    // log psi alone, for a caller that reads it: 16 states per tile.  (An exact
+    // enumeration's |psi|^2 weights, which the SR solve amplifies, come in FP64
+    // from a group of lanes per state, whose sums keep their order.)
     if (logpsi && !obs && !Tout && !ratio && !c->pf_rows && logpsi_tables_fit(c->nsymm, c->N))
         return run_logpsi<R>(c, d_states, n, logpsi);
     if constexpr (sizeof(R) == 4) {
         // sample sets in FP32: the tanh rows and observables through the wave
         // sampler's tables (basic RBM: k_eloc's observables), log psi by
-        // k_logpsi.  FP64 sample sets keep the lane-group evaluation: its sums'
-        // order reaches the SR solve, which amplifies a change of rounding.
-        if (Tout == c->d_T && obs == c->d_obs && !ratio && wave_ok(c) && (!logpsi || logpsi_tables_fit(c->nsymm, c->N))) {
+        // k_logpsi, where that is faster.  FP64 sample sets keep the lane-group
+        // evaluation: its sums' order reaches the SR solve, which amplifies a
+        // change of rounding.
+        if (Tout == c->d_T && obs == c->d_obs && !ratio && wave_ok(c) && eval_wave_faster(c, n) &&
+            (!logpsi || logpsi_tables_fit(c->nsymm, c->N))) {
             SampArgs<float> w = samp_args<float>(c, 0, 512, n, 0);
             const int K = (c->H + 63) / 64;
             w.npair = c->nsymm > 1 ? c->npair : 0;
@@ -2329,6 +2360,7 @@ int rbmgpu_create(const rbmgpu_config* cfg, rbmgpu_ctx** out) {
             for (int b = 0; b < npb; b++)
                 if ((c->pb[2 * b] == x && c->pb[2 * b + 1] == y) || (c->pb[2 * b] == y && c->pb[2 * b + 1] == x)) {
                     tbond[t] = (int16_t)b;
+                    c->n_pair_terms += term_slot[t] >= 0;
                     break;
                 }
         }

@@ -59,3 +59,27 @@ def test_eval_wave_large_visible_bias(n, alpha, c):
     e, got = o.eloc(st), g.get_samples()[1][:, 0]
     assert np.all(np.isfinite(got))
     assert np.max(np.abs(got - e)) <= 1e-4 * np.abs(e).max()
+
+
+# set sizes on both sides of the lines between the evaluations: groups of lanes
+# below, the wave sampler's tables above
+@pytest.mark.parametrize("model,n,rbm,alpha,extra,line",
+                         [("toric", 3, "symmetry", 4, "", 16384), ("kitaev", 3, "symmetry", 2, "helper_strength = 0.2\n", 5120),
+                          ("kitaev", 6, "symmetry", 1, "helper_strength = 0.2\n", 8192), ("toric", 4, "basic", 2, "", 5120),
+                          ("kitaev", 4, "basic", 3, "", 4096), ("kitaev", 5, "basic", 2, "", 512),
+                          ("kitaev", 4, "basic", 1, "helper_strength = 0.2\n", 8192)])
+def test_eval_wave_lines(model, n, rbm, alpha, extra, line):
+    print(f"[gpu-test] eval_wave line {model} {n} {rbm} alpha={alpha} {extra.strip()} {line}", flush=True)
+    rng = np.random.default_rng(n * 10 + alpha)
+    spec = ini(model, n, rbm=rbm, alpha=alpha, extra="[model]\n" + extra if extra else "")
+    m, o = rbmgpu.Model(spec), po.Oracle(spec)
+    p = random_params(rng, m.P, 0.1)
+    o.set_params(p)
+    g = m.gpu(precision=32)
+    g.set_params(p)
+    st = po.random_states(rng, 64, m.N)
+    e = o.eloc(st)
+    for S in (line - 1, line):
+        g.load_samples(np.resize(st, (S, st.shape[1])))
+        got = g.get_samples()[1][:, 0]
+        assert np.max(np.abs(got - np.resize(e, S))) <= 1e-4 * (1 + np.abs(e).max()), S
