@@ -26,8 +26,8 @@ HIPFLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",
             "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 CXXFLAGS = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-sign-compare"]
 
-GPU_SOURCES = ["kern_f32.hip", "kern_f64.hip", "kern_struct.hip", "kern_logpsi.hip", "kern_learn.hip", "kern_eloc.hip",
-               "kern_dense.hip", "kern_wave.hip", "rbmgpu_host.hip"]
+GPU_SOURCES = ["kern_f64.hip", "kern_f32.hip", "kern_pf_sample.hip", "kern_pf_eval.hip", "kern_struct.hip",
+               "kern_logpsi.hip", "kern_learn.hip", "kern_eloc.hip", "kern_dense.hip", "kern_wave.hip", "rbmgpu_host.hip"]
 HOST_SOURCES = ["lattice.cpp", "model.cpp", "ini.cpp", "setup.cpp", "optim.cpp", "capi.cpp"]
 DRIVER_SOURCES = ["main.cpp", "adapters.cpp"]
 

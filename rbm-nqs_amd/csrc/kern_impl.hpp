@@ -811,8 +811,13 @@ __global__ void __launch_bounds__(PF && sizeof(R) == 4 ? kPfBlock : 256) k_sampl
 // ---------------------------------------------------------- eval states --
 // one group per host-given state: theta from scratch, tanh, optionally
 // log psi, local observables and the psi ratio for given flips
-template <typename R, int L, int K, bool PF>
-__global__ void __launch_bounds__(256) k_eval(EvalArgs<R> a) {
+// WS: wavefronts per SIMD that the registers have to leave room for.  One, but
+// with the Pfaffian factor in FP64 and one unit per lane two where there are
+// states and LDS for them (256 registers instead of 290; Kitaev 3x3 alpha = 1,
+// 32 768 states: 4010 -> 2841 us; alpha = 3, where LDS holds one block per CU:
+// 4060 us with one, 4511 with two)
+template <typename R, int L, int K, bool PF, int WS>
+__global__ void __launch_bounds__(256, WS) k_eval(EvalArgs<R> a) {
     extern __shared__ __align__(16) char smem[];
     const Dims d = a.d;
     Lds<R> l = stage<R>(d, a.t, a.T, a.pb, smem);
@@ -826,7 +831,8 @@ __global__ void __launch_bounds__(256) k_eval(EvalArgs<R> a) {
     U.init(d, ln);
     U.from_state(d, l, a.t.hb, st);
     cplx<R> pv[16];
-    if constexpr (PF) pf_fresh(l.pf, st, ln, pv);
+    if constexpr (PF)  // (log psi alone does not need the inverse)
+        if (a.Opf || a.obs || a.ratio) pf_fresh(l.pf, st, ln, pv);
     if (a.Tout) {
 #pragma unroll
         for (int u = 0; u < K; u++)

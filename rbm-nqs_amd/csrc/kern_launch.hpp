@@ -20,17 +20,19 @@ static hipError_t sample_one(const SampArgs<R>& a, int block, hipStream_t st) {
     hipLaunchKernelGGL((k_sample<R, L, K, PF>), dim3(grid), dim3(block), lds, st, a);
     return hipGetLastError();
 }
-template <typename R, int L, int K, bool PF>
+template <typename R, int L, int K, bool PF, int WS = 1>
 static hipError_t eval_one(const EvalArgs<R>& a, int block, hipStream_t st) {
     int64_t threads = a.n * L;
     int grid = (int)((threads + block - 1) / block);
     size_t lds = lds_bytes<R>(a.d);
+    if constexpr (PF && sizeof(R) == 8 && K == 1 && WS == 1)
+        if (a.n > 1024 && (int)(163840 / lds) * (block / 64) > 4) return eval_one<R, L, K, PF, 2>(a, block, st);
     if (lds > 65536) {
-        hipError_t e = hipFuncSetAttribute((const void*)k_eval<R, L, K, PF>,
+        hipError_t e = hipFuncSetAttribute((const void*)k_eval<R, L, K, PF, WS>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL((k_eval<R, L, K, PF>), dim3(grid), dim3(block), lds, st, a);
+    hipLaunchKernelGGL((k_eval<R, L, K, PF, WS>), dim3(grid), dim3(block), lds, st, a);
     return hipGetLastError();
 }
 
@@ -40,16 +42,37 @@ static hipError_t eval_one(const EvalArgs<R>& a, int block, hipStream_t st) {
 // shapes with a Pfaffian instance: one chain per wavefront
 #define PF_SHAPES(X) X(64, 1) X(64, 2) X(64, 4) X(64, 8)
 
+// The Pfaffian instances of the sampler and of the evaluation are translation
+// units of their own (kern_pf_sample.hip, kern_pf_eval.hip): together, the
+// functions that they share are called from both and no longer inlined where
+// they are large, which puts the units and the inverse in scratch memory (8
+// units per lane: 760 bytes a lane instead of 40).
 template <typename R>
-hipError_t launch_sample(const SampArgs<R>& a, Shape s, int block, hipStream_t st) {
-    if (a.d.pf_rows) {
-        if (block != 64 * a.d.waves) return hipErrorInvalidValue;
+hipError_t launch_sample_pf(const SampArgs<R>& a, Shape s, int block, hipStream_t st) {
+    if (block != 64 * a.d.waves) return hipErrorInvalidValue;
 #define X(L_, K_) \
     if (s.L == L_ && s.K == K_) return sample_one<R, L_, K_, true>(a, block, st);
-        PF_SHAPES(X)
+    PF_SHAPES(X)
 #undef X
-        return hipErrorInvalidValue;
-    }
+    return hipErrorInvalidValue;
+}
+template <typename R>
+hipError_t launch_eval_pf(const EvalArgs<R>& a, Shape s, int block, hipStream_t st) {
+    if (block != 64 * a.d.waves) return hipErrorInvalidValue;
+#define X(L_, K_) \
+    if (s.L == L_ && s.K == K_) return eval_one<R, L_, K_, true>(a, block, st);
+    PF_SHAPES(X)
+#undef X
+    return hipErrorInvalidValue;
+}
+extern template hipError_t launch_sample_pf<float>(const SampArgs<float>&, Shape, int, hipStream_t);
+extern template hipError_t launch_sample_pf<double>(const SampArgs<double>&, Shape, int, hipStream_t);
+extern template hipError_t launch_eval_pf<float>(const EvalArgs<float>&, Shape, int, hipStream_t);
+extern template hipError_t launch_eval_pf<double>(const EvalArgs<double>&, Shape, int, hipStream_t);
+
+template <typename R>
+hipError_t launch_sample(const SampArgs<R>& a, Shape s, int block, hipStream_t st) {
+    if (a.d.pf_rows) return launch_sample_pf<R>(a, s, block, st);
 #define X(L_, K_) \
     if (s.L == L_ && s.K == K_) return sample_one<R, L_, K_, false>(a, block, st);
     RBM_SHAPES(X)
@@ -58,14 +81,7 @@ hipError_t launch_sample(const SampArgs<R>& a, Shape s, int block, hipStream_t s
 }
 template <typename R>
 hipError_t launch_eval(const EvalArgs<R>& a, Shape s, int block, hipStream_t st) {
-    if (a.d.pf_rows) {
-        if (block != 64 * a.d.waves) return hipErrorInvalidValue;
-#define X(L_, K_) \
-    if (s.L == L_ && s.K == K_) return eval_one<R, L_, K_, true>(a, block, st);
-        PF_SHAPES(X)
-#undef X
-        return hipErrorInvalidValue;
-    }
+    if (a.d.pf_rows) return launch_eval_pf<R>(a, s, block, st);
 #define X(L_, K_) \
     if (s.L == L_ && s.K == K_) return eval_one<R, L_, K_, false>(a, block, st);
     RBM_SHAPES(X)
