@@ -19,6 +19,7 @@
 
 #include "../../include/rbmgpu.h"
 #include "kern_api.hpp"
+#include "ofree_index.hpp"
 
 using namespace rbmgpu;
 using zd = std::complex<double>;
@@ -75,7 +76,7 @@ struct rbmgpu_ctx {
     // ofree: other basic RBMs (FP64, keep_o, Pfaffian factor); moments and S.x
     // form O's entries from the states and tanh rows (k_sx_ofree,
     // k_o_partial), the O matrix is built when something reads it
-    // (rbmgpu_get_samples, the explicit S)
+    // (rbmgpu_get_samples, the explicit S, solves on small sets: sx_from_O)
     bool ofree = false;
     bool o_built = false;  // d_O holds the current sample set (ofree)
     int64_t o_cap = 0;     // samples d_O has room for (ofree)
@@ -630,17 +631,49 @@ int run_build_O(rbmgpu_ctx* c) {
     return enqueue_build_O<R>(c);
 }
 
+// ofree: whether a solve on S samples is faster over the O matrix, built once,
+// than with its entries formed in every product (the same products and sums
+// either way).  As long as O stays in the caches, k_sx_partial's loads cost less
+// than k_sx_ofree's setup per row, most of all with the Pfaffian block, which
+// both read.  Set, moments and 80 CG iterations, relative to the
+// moments read from O too, entries formed / over O:
+//   FP64: rows of up to 512 entries while O has at most 24 MB (Kitaev 2x2
+//     alpha = 3: 22 MB 1.07 / 1.03, 72 MB 0.89 / 1.00); longer rows never
+//     (3x3 alpha = 2, 2000 samples: 0.74 / 1.00)
+//   FP32: 48 MB (3x3 alpha = 1: 17 MB 1.07 / 0.98, 58 MB 0.95 / 0.97), N > 32
+//     160 MB (5x5: 125 MB 1.06 / 0.98), N = 32 with tanh by row broadcasts never
+//     (4x4 alpha = 1: 9 MB 0.95 / 1.01)
+//   Pfaffian FP32: 160 MB (4x4 alpha = 2: 108 MB 0.93 / 0.84, 359 MB 0.69 / 0.79)
+//   Pfaffian FP64: one pair per lane 160 MB (2x2 alpha = 1: 104 MB 1.06 / 0.98),
+//     up to 512 entries 32 MB (2x2 alpha = 4: 10 MB 1.20 / 0.99, 31 MB 1.01 / 1.01),
+//     longer 16 MB (3x3 alpha = 2: 12 MB 1.02 / 0.96, 24 MB 0.87 / 0.95), N = 32
+//     never (4x4 alpha = 1, 200 samples: 0.89 / 0.95)
+bool sx_from_O(const rbmgpu_ctx* c, int64_t S) {
+    if (!c->ofree) return false;
+    const int mode = of_mode(c->N, c->na);
+    int mb;
+    if (c->prec == RBMGPU_FP32)
+        mb = c->pf_rows ? 160 : mode == kOfB32 ? 0 : mode == kOfWide ? 160 : 48;
+    else if (c->pf_rows)
+        mb = c->ld <= 128 ? 160 : c->ld <= 512 ? 32 : mode == kOfB32 ? 0 : 16;
+    else
+        mb = c->ld <= 512 ? 24 : 0;
+    return S * c->ld * 2 * (int64_t)rsize(c) <= (int64_t)mb * 1000000;
+}
+
+// a training epoch's graph holds O's address
+bool train_reads_O(const rbmgpu_ctx* c) { return c->train_dense == 1 || sx_from_O(c, c->n_samples); }
+
 // ofree: the O matrix of the current sample set, if it is not there yet
 int ensure_O(rbmgpu_ctx* c) {
     rbmgpu_ctx* ctx = c;
     if (!c->ofree || c->o_built || c->S == 0) return 0;
     if (c->S > c->o_cap) {
         c->o_cap = 0;
-        // captured epochs hold O's address only where they build S from it:
-        // the others stay
+        // captured epochs that do not read O hold no address of it and stay
         const uint64_t gen = c->gen;
         if (int rc = dalloc(ctx, &c->d_O, c->S * c->ld * 2 * rsize(c))) return rc;
-        if (c->train_dense != 1) c->gen = gen;
+        if (!train_reads_O(c)) c->gen = gen;
         c->o_cap = c->S;
     }
     if (int rc = c->prec == RBMGPU_FP32 ? enqueue_build_O<float>(c) : enqueue_build_O<double>(c)) return rc;
@@ -1424,7 +1457,7 @@ SxArgs<R> sx_args(rbmgpu_ctx* c, const double* x, double* y, double r1, double r
     a.part = (cplx<R>*)c->d_sxpart;
     a.y = y;
     a.status = st;
-    if (c->ofree) {
+    if (c->ofree && !(c->o_built && sx_from_O(c, c->S))) {
         a.N = c->N;
         a.M = c->na;
         a.P_rbm = (int)c->P_rbm;
@@ -2134,6 +2167,8 @@ int train_body(rbmgpu_ctx* c, int64_t n_cg) {
         const double* reg = reinterpret_cast<const double*>(reinterpret_cast<const char*>(c->d_par) +
                                                             offsetof(DevPar, reg));
         if (int rc = build_S(c, 0, 0, 0, 0, reg)) return rc;
+    } else if (sx_from_O(c, c->S)) {
+        if (int rc = ensure_O(c)) return rc;
     }
     if (int rc = train_mv(c, c->d_x, c->d_Ap, nullptr, false)) return rc;
     hipLaunchKernelGGL(k_cg_init, dim3(1), dim3(1024), 0, c->stream, c->d_b, c->d_Ap, c->d_r, c->d_p, (int)c->P,
@@ -2579,7 +2614,7 @@ int rbmgpu_train_epoch(rbmgpu_ctx* c, uint32_t epoch, const rbmgpu_sr_params* sp
         if (ex) {
             HIPCK(hipGraphLaunch(ex, c->stream));
             epoch_state(c);
-            c->o_built = c->train_dense == 1;  // O only if S was built from it
+            c->o_built = c->ofree && train_reads_O(c);
             if (int rc = ensure_sx(c)) return rc;  // this set's layout, for train_more
         } else {
             // this epoch runs eagerly (allocating what it needs), then the
@@ -3005,8 +3040,11 @@ int rbmgpu_sr_solve_ex(rbmgpu_ctx* c, int32_t method, const double* b, double* x
         return 0;
     }
     const bool dense = method == RBMGPU_SOLVE_CG_SINGLE;
-    if (dense)
+    if (dense) {
         if (int rc = build_S(c, r1, r2, rd, 0)) return rc;
+    } else if (sx_from_O(c, c->S)) {
+        if (int rc = ensure_O(c)) return rc;
+    }
     // cg_solver.cpp:48-60: max_iter = min(2P, max_iter), 0 -> 2P; rtol 0 -> 1e-16
     int64_t mi = std::min<int64_t>(2 * c->P, max_iter);
     if (mi == 0) mi = 2 * c->P;
