@@ -436,11 +436,11 @@ template <typename R>
 hipError_t launch_build_O(const OArgs<R>& a, hipStream_t st);
 template <typename R>
 hipError_t launch_o_partial(const MomArgs<R>& a, int blocks, hipStream_t st);
-// block partials of S.x over the materialised O (k_sx_partial); the caller
+// block partials of S.x over the materialised O (k_sx_partial), or with a.T from
+// the tanh rows (k_sx_ofree); the caller
 // finishes the product with launch_sx_colsum
 template <typename R>
-hipError_t launch_sx(const SxArgs<R>& a, int blocks, hipStream_t st, hipEvent_t e0 = nullptr,
-                     hipEvent_t e1 = nullptr);
+hipError_t launch_sx(const SxArgs<R>& a, int blocks, hipStream_t st);
 // ZM (P <= 64*ZM) supported by launch_sx
 int sx_max_params();
 // whether launch_sx and launch_o_partial can form O's entries from the tanh

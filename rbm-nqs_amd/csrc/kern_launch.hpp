@@ -1,8 +1,6 @@
 // kern_launch.hpp -- launchers that dispatch the runtime launch shape to the
 // compiled template instances; included once per precision.
 #pragma once
-#include <hip/hip_ext.h>
-
 #include "kern_impl.hpp"
 
 namespace rbmgpu {
@@ -131,19 +129,19 @@ template <typename R, int ZM, int WAVES>
 static hipError_t sx_ofree(const SxArgs<R>& a, int blocks, hipStream_t st) {
     const bool pf = a.P > a.P_rbm;
     const int mode = of_mode(a.N, a.M);
-    // N >= 32 has P >= 1088, in blocks of 4 waves; the Pfaffian factor N <= 32
-    if constexpr (WAVES == 4) {
+    // B32 has P >= 1088 (more than 8 pairs per lane); the Pfaffian factor N <= 32
+    if constexpr (ZM > 8)
         if (mode == kOfB32)
             return pf ? sx_ofree_go<R, ZM, WAVES, kOfB32, true>(a, blocks, st)
                       : sx_ofree_go<R, ZM, WAVES, kOfB32, false>(a, blocks, st);
+    if constexpr (WAVES == 4)
         if (mode == kOfWide) return pf ? hipErrorInvalidValue : sx_ofree_go<R, ZM, WAVES, kOfWide, false>(a, blocks, st);
-    }
     if (mode != kOfN32) return hipErrorInvalidValue;
     return pf ? sx_ofree_go<R, ZM, WAVES, kOfN32, true>(a, blocks, st)
               : sx_ofree_go<R, ZM, WAVES, kOfN32, false>(a, blocks, st);
 }
 template <typename R, int ZM, int WAVES = 4>
-static hipError_t sx_one(const SxArgs<R>& a, int blocks, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
+static hipError_t sx_one(const SxArgs<R>& a, int blocks, hipStream_t st) {
     if (a.T) return sx_ofree<R, ZM, WAVES>(a, blocks, st);
     size_t lds = 2 * (size_t)a.ld * sizeof(cplx<R>);
     if (lds > 65536) {
@@ -151,21 +149,17 @@ static hipError_t sx_one(const SxArgs<R>& a, int blocks, hipStream_t st, hipEven
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
     }
-    if (e0 || e1)
-        hipExtLaunchKernelGGL((k_sx_partial<R, ZM, WAVES>), dim3(blocks), dim3(64 * WAVES), (uint32_t)lds, st, e0,
-                              e1, 0u, a);
-    else
-        hipLaunchKernelGGL((k_sx_partial<R, ZM, WAVES>), dim3(blocks), dim3(64 * WAVES), lds, st, a);
+    hipLaunchKernelGGL((k_sx_partial<R, ZM, WAVES>), dim3(blocks), dim3(64 * WAVES), lds, st, a);
     return hipGetLastError();
 }
 template <typename R>
-hipError_t launch_sx(const SxArgs<R>& a, int blocks, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
-    if (a.ld <= 128 * 2) return sx_one<R, 2, 16>(a, blocks, st, e0, e1);
-    if (a.ld <= 128 * 4) return sx_one<R, 4, 16>(a, blocks, st, e0, e1);
-    if (a.ld <= 128 * 8) return sx_one<R, 8>(a, blocks, st, e0, e1);
-    if (a.ld <= 128 * 12) return sx_one<R, 12>(a, blocks, st, e0, e1);
-    if (a.ld <= 128 * 18) return sx_one<R, 18>(a, blocks, st, e0, e1);
-    if (a.ld <= 128 * 24) return sx_one<R, 24>(a, blocks, st, e0, e1);
+hipError_t launch_sx(const SxArgs<R>& a, int blocks, hipStream_t st) {
+    if (a.ld <= 128 * 2) return sx_one<R, 2, 16>(a, blocks, st);
+    if (a.ld <= 128 * 4) return sx_one<R, 4, 16>(a, blocks, st);
+    if (a.ld <= 128 * 8) return sx_one<R, 8>(a, blocks, st);
+    if (a.ld <= 128 * 12) return sx_one<R, 12>(a, blocks, st);
+    if (a.ld <= 128 * 18) return sx_one<R, 18>(a, blocks, st);
+    if (a.ld <= 128 * 24) return sx_one<R, 24>(a, blocks, st);
     return hipErrorInvalidValue;
 }
 
@@ -188,6 +182,6 @@ hipError_t launch_sx_colsum(const SxArgs<R>& a, hipStream_t st) {
     template hipError_t launch_eval<R>(const EvalArgs<R>&, Shape, int, hipStream_t);      \
     template hipError_t launch_build_O<R>(const OArgs<R>&, hipStream_t);                  \
     template hipError_t launch_o_partial<R>(const MomArgs<R>&, int, hipStream_t);         \
-    template hipError_t launch_sx<R>(const SxArgs<R>&, int, hipStream_t, hipEvent_t, hipEvent_t);
+    template hipError_t launch_sx<R>(const SxArgs<R>&, int, hipStream_t);
 
 }  // namespace rbmgpu

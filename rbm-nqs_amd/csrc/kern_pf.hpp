@@ -365,12 +365,11 @@ __device__ inline cplx<double> pf_logpf(const PfLds<R>& l, const uint64_t* st, i
     return {lre, lim};
 }
 
-// Pfaffian of the 2m x 2m skew matrix G (row-major, stride 16): closed forms
-// for m <= 2, Parlett-Reid by one lane otherwise (uniform result)
+// Pfaffian of the 2m x 2m skew matrix G (row-major, stride 16), m > 2 (the
+// closed forms of one and two flips are pf_ratio2's), by Parlett-Reid in one
+// lane (uniform result)
 template <typename R>
 __device__ inline cplx<R> small_pf(cplx<R>* G, int m, int lane) {
-    if (m == 1) return G[1];
-    if (m == 2) return G[1] * G[2 * 16 + 3] - G[2] * G[1 * 16 + 3] + G[3] * G[1 * 16 + 2];
     cplx<R> pf{1, 0};
     if (lane == 0) {
         const int n = 2 * m;
@@ -598,7 +597,7 @@ __device__ inline cplx<R> pf_ratio(const PfLds<R>& l, const cplx<R> (&v)[16], co
             }
     wave_sync();
     cplx<R> pf = small_pf(l.G, m, lane);
-    if (m > 2) wave_sync();
+    wave_sync();
     bool neg = ((m * (m + 1) / 2) & 1) != 0;
     return neg ? cplx<R>{-pf.re, -pf.im} : pf;
 }
