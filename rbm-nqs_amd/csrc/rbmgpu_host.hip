@@ -2193,7 +2193,18 @@ int train_more(rbmgpu_ctx* c, int64_t n_cg) {
 // per iteration a P x P complex mat-vec fused with the CG step (~8 us)
 // against a pass over O per iteration (S ld 8 or 16 bytes at ~6 TB/s plus
 // ~15 us of launches); the same trade as the reference's cg-dynamic
-// (cg_solver.cpp:31-46), with this device's rates
+// (cg_solver.cpp:31-46), with this device's rates.
+//
+// Basic machines that form O's entries in the product (sx_from_O false) need
+// less than that pass, and all of them build O for S in every epoch.  Where the
+// line lies has been measured for them (epoch in us, FP64, explicit S /
+// matrix-free): P = 80, 16 384 samples 1186 / 2003; P = 360, 16 384 2676 / 3715,
+// 65 536 4704 / 5155, 262 144 15288 / 14314; P = 702, 4096 2776 / 3567, 16 384
+// 4163 / 4933, 65 536 9048 / 9483; P = 1044, 16 384 6882 / 5823; P = 1088, 16 384
+// 6922 / 4914.  The rates below choose the faster one but for P = 360 at 262 144
+// (7 % lost) and P = 702 from 16 384 on (5 to 16 %).  They stay as they are: the
+// two products round differently, which an ill-conditioned solve carries into
+// the weights of a run.
 int decide_train_dense(const rbmgpu_ctx* c, int64_t max_iter) {
     if (c->structured) return 0;  // no O matrix
     const double S = (double)c->n_samples, P = (double)c->P, ld = (double)c->ld;

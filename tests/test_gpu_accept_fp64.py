@@ -1,6 +1,6 @@
 """The FP64 sampler's acceptance (u against the group product of the lanes'
-|p|^2 as mantissa and exponent, visible bias on u's side) and its incremental
-tanh, against the oracle state for state: every group width with one and with
+|p|^2 as mantissa and exponent, visible bias on u's side) and its moves,
+against the oracle state for state: every group width with one and with
 several units per lane, padded lanes, two state words, symmetric RBMs, and
 visible biases and weights whose ratios span hundreds of binary orders.  E_loc
 of the kept samples to 1e-10 of the largest, as in test_gpu_parity.py: it is
