@@ -705,9 +705,9 @@ __global__ void __launch_bounds__(1024) k_sample_wave(SampArgs<float> a) {
 // and tanh from scratch, tanh rows, and the local observables unless a.obs is
 // null.  The blocks that fit the CUs walk the states, so the pair tables and
 // entry factors are built once per resident block.  Kitaev 6x6 symmetric
-// alpha = 4, 65 536 states: 5670 us by the lane-group evaluation (each flipped
-// site composed per unit, one term's product reduced at a time), 1990 us; bound
-// by the vector pipe and the LDS reads of the terms' records.
+// alpha = 4, 65 536 states: 5700 us by the lane-group evaluation (each flipped
+// site composed per unit, one term's product reduced at a time), 2090 us; bound
+// by VALU issue (0.89 of the cycles).
 template <int K, bool SYM>
 __global__ void __launch_bounds__(kWaveEvalBlock) k_eval_wave(SampArgs<float> a) {
     extern __shared__ __align__(16) char smem[];

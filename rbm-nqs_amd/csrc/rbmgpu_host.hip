@@ -635,8 +635,8 @@ int run_build_O(rbmgpu_ctx* c) {
 // than with its entries formed in every product (the same products and sums
 // either way).  As long as O stays in the caches, k_sx_partial's loads cost less
 // than k_sx_ofree's setup per row, most of all with the Pfaffian block, which
-// both read.  Set, moments and 80 CG iterations, relative to the
-// moments read from O too, entries formed / over O:
+// both read.  Set, moments and 80 CG iterations, relative to O built
+// with every set, entries formed / over O built for the solve:
 //   FP64: rows of up to 512 entries while O has at most 24 MB (Kitaev 2x2
 //     alpha = 3: 22 MB 1.07 / 1.03, 72 MB 0.89 / 1.00); longer rows never
 //     (3x3 alpha = 2, 2000 samples: 0.74 / 1.00)
