@@ -55,8 +55,9 @@ __device__ inline T* lds_copy(char*& at, const T* src, size_t n) {
 }
 
 // stage the weight tables, visible biases, proposal bonds, local-operator
-// tables and symmetry permutations into LDS (layout of lds_bytes)
-template <typename R>
+// tables and symmetry permutations into LDS (layout of lds_bytes); with PF the
+// Pfaffian tables and the waves' scratch
+template <typename R, bool PF = false>
 __device__ inline Lds<R> stage(const Dims& d, const Tabs<R>& t, const Terms& T, const int32_t* pb,
                                char* smem) {
     const size_t nw = (size_t)d.N * d.n_alpha;
@@ -68,7 +69,7 @@ __device__ inline Lds<R> stage(const Dims& d, const Tabs<R>& t, const Terms& T, 
     l.Wl = d.w_lds ? lds_copy(at, t.W, nw) : reinterpret_cast<const cplx<R>*>(at);
     l.rb = lds_copy(at, t.rb, d.N);
     l.pf = {};
-    if (d.pf_rows) {
+    if constexpr (PF) {
         l.pf.fs = lds_copy(at, t.fs, 4 * (size_t)d.pf_rows);
         const size_t sw = pf_scratch<R>(d.N, d.pf_rows, d.pf_full);
         at = smem + ((at - smem + 15) & ~(ptrdiff_t)15);
@@ -93,7 +94,7 @@ __device__ inline Lds<R> stage(const Dims& d, const Tabs<R>& t, const Terms& T, 
         l.Tl.rowbase = lds_copy(at, T.rowbase, d.n_terms);
     }
     l.pb = lds_copy(at, pb, 2 * (size_t)d.npb);
-    if (d.pf_rows) l.pf.bs = lds_copy(at, t.bs, (size_t)d.N * d.N);
+    if constexpr (PF) l.pf.bs = lds_copy(at, t.bs, (size_t)d.N * d.N);
     if (d.t_lds) {
         l.Tl.sites = lds_copy(at, T.sites, 8 * (size_t)d.n_terms);
         l.Tl.mask = lds_copy(at, T.mask, d.n_ent);
@@ -657,8 +658,8 @@ __device__ inline void eval_obs(const Dims& d, const Lds<R>& l, const Units<R, L
 // steps the local observables and tanh(theta) of the sample are written.
 // A chain is one dependent sequence of proposals, so with few chains the sampler
 // is bound by a proposal's latency: in FP64 the decision takes no logarithm
-// (toric 4x4 symmetric, 64 chains, 450 sweeps: epoch 17.9 -> 16.0 ms; basic,
-// 4096 chains x 164 sweeps: 57.8 -> 57.1 ms).
+// (toric 4x4 symmetric, 64 chains, 450 sweeps: epoch 17.9 -> 15.7 ms; basic,
+// 4096 chains x 164 sweeps: 57.8 -> 56.2 ms).
 // With the Pfaffian factor in FP32 up to 8 chains share a block's tables: its
 // LDS lets one block per CU run (Kitaev 4x4), as two wavefronts per SIMD of 256
 // registers; in FP64 one of 512 registers.
@@ -666,7 +667,7 @@ template <typename R, int L, int K, bool PF>
 __global__ void __launch_bounds__(PF && sizeof(R) == 4 ? kPfBlock : 256) k_sample(SampArgs<R> a) {
     extern __shared__ __align__(16) char smem[];
     const Dims d = a.d;
-    Lds<R> l = stage<R>(d, a.t, a.T, a.pb, smem);
+    Lds<R> l = stage<R, PF>(d, a.t, a.T, a.pb, smem);
     int gtid = blockIdx.x * blockDim.x + threadIdx.x;
     int chain = gtid / L, ln = gtid % L;
     if (chain >= a.n_chains) return;
@@ -741,15 +742,18 @@ __global__ void __launch_bounds__(PF && sizeof(R) == 4 ? kPfBlock : 256) k_sampl
             cplx<R> p;
             int pe;
             U.ratio12(d, l, f0, s0, f1, s1, p, pe);
-            R bre = (-2 * s0) * l.rb[f0].re;
-            if (f1 >= 0) bre += (-2 * s1) * l.rb[f1].re;
-            constexpr R kBias = (R)2.8853900817779268;  // 2 / ln 2: visible-bias term 2 Re(-2 sum sigma_f c_f)
+            // visible-bias term 2 Re(-2 sum sigma_f c_f), base 2
+            auto bias = [&]() __attribute__((always_inline)) {
+                R bre = (-2 * s0) * l.rb[f0].re;
+                if (f1 >= 0) bre += (-2 * s1) * l.rb[f1].re;
+                return (R)2.8853900817779268 * bre;  // 2 / ln 2
+            };
             bool take;
             if constexpr (sizeof(R) == 8) {
                 // u < |psi'/psi|^2 as u / 2^bias < group product of the lanes'
                 // |p|^2, as mantissa and exponent, so that the product stays in
                 // range whatever the lanes' factors are
-                const R b2 = kBias * bre, bt = b2 > 1e6 ? 1e6 : b2 < -1e6 ? -1e6 : b2, bi = __builtin_rint(bt);
+                const R b2 = bias(), bt = b2 > 1e6 ? 1e6 : b2 < -1e6 ? -1e6 : b2, bi = __builtin_rint(bt);
                 const R lhs = uu * M<R>::exp2(bi - bt);
                 const R n2 = norm2(p);
                 R pm = frexp_m(n2);
@@ -768,7 +772,7 @@ __global__ void __launch_bounds__(PF && sizeof(R) == 4 ? kPfBlock : 256) k_sampl
                 // log2 |psi'/psi|^2: group sum of the lanes' log2 |p|^2, plus the bias
                 R lp = M<R>::log2(norm2(p)) + (R)(2 * pe);
                 R lr2 = group_sum<L>(lp);
-                lr2 += kBias * bre;
+                lr2 += bias();
                 if constexpr (PF) {
                     cplx<R> q = pf_ratio2<R, true>(l.pf, pv, st, __builtin_amdgcn_readfirstlane(f0),
                                                    __builtin_amdgcn_readfirstlane(f1), ln, pp);
@@ -820,7 +824,7 @@ template <typename R, int L, int K, bool PF, int WS>
 __global__ void __launch_bounds__(256, WS) k_eval(EvalArgs<R> a) {
     extern __shared__ __align__(16) char smem[];
     const Dims d = a.d;
-    Lds<R> l = stage<R>(d, a.t, a.T, a.pb, smem);
+    Lds<R> l = stage<R, PF>(d, a.t, a.T, a.pb, smem);
     int gtid = blockIdx.x * blockDim.x + threadIdx.x;
     int64_t g = gtid / L;
     int ln = gtid % L;
